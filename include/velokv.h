@@ -175,7 +175,9 @@ int vk_ctx_set_decode_kernel(vk_ctx* ctx, int kind);
  * split its blocks evenly and combine split pairs in LDS: no merge launch and no
  * workspace; fp16 / int8 KV, at most 256 sequences, else stream-K) or VK_SCHED_AUTO (stream-K
  * unless vk_decode_args.sum_context_len says the batch is uniform, or the VALU
- * family was requested). A nonzero partition_tokens always uses fixed partitions. No
+ * family was requested; a small batch whose lengths' sum is known, or of one
+ * sequence, runs the workgroup split, one workgroup per (sequence, KV head), or
+ * per partition of the longer contexts with a merge launch). A nonzero partition_tokens always uses fixed partitions. No
  * reference counterpart. */
 #define VK_SCHED_AUTO 0
 #define VK_SCHED_SPLIT 1
@@ -321,7 +323,10 @@ typedef struct vk_decode_args {
   int64_t sum_context_len;    /* host sum of context_lens if known, else 0: with
                                  VK_SCHED_AUTO a batch whose sum is within 3 % of
                                  n_seqs * max_context_len runs fixed partitions,
-                                 any other (or unknown) batch runs stream-K    */
+                                 any other (or unknown) batch runs stream-K, and
+                                 a small batch a workgroup split sized by it. It
+                                 steers the plan only: any context_lens up to
+                                 max_context_len are computed whatever it says */
 } vk_decode_args;
 
 /* Bytes of workspace vk_paged_decode needs for these arguments. */
@@ -339,8 +344,9 @@ typedef struct vk_decode_plan {
   int32_t schedule;            /* VK_SCHED_SPLIT, _STREAM, _WORKGROUP or _PACKED       */
   int32_t wg_waves;            /* waves per workgroup of the attention launch
                                   (workgroup split, packed split, stream-K)          */
-  int32_t partition_tokens;    /* fixed partitions: tokens per partition               */
-  int32_t max_partitions;      /* fixed partitions: partitions of the longest context  */
+  int32_t partition_tokens;    /* fixed partitions, and a workgroup split in partitions:
+                                  tokens per partition                               */
+  int32_t max_partitions;      /* ... partitions of the longest context (else 0)       */
   int32_t n_workers;           /* stream-K: workers (one wave each, wg_waves of them
                                   per workgroup); packed: workgroups                 */
   int32_t max_blocks_per_wave; /* the most blocks one wave can walk (<= 256)           */
@@ -368,8 +374,9 @@ int vk_paged_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* s
  * slots followed by vk_paged_decode, bit for bit, and so do the outputs except
  * under the workgroup split, whose folding wave takes a few blocks fewer (the
  * outputs then agree to fp32 rounding of a different split). Over VK_KV_I8_BLK pools under the
- * workgroup-split or stream-K schedule, and over VK_KV_F16 pools under
- * stream-K, the decode launch appends the tokens itself (the
+ * workgroup-split or stream-K schedule, over VK_KV_F16 pools for ragged batches under
+ * either, and over any pool for one sequence under the workgroup split, the decode
+ * launch appends the tokens itself (the
  * wave that holds a sequence's last block applies the append rule to it before
  * loading it; two sequences whose new tokens share a block are reported,
  * VK_MISUSE_BLK_SPLIT_RUN); otherwise the append kernel runs first, with the

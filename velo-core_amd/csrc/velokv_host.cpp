@@ -311,7 +311,7 @@ extern "C" int vk_ctx_create(int device, const char* code_object_path, vk_ctx** 
       names.push_back(decode_mfma_name(kv, 3, qt));
       names.push_back(decode_mfma_name(kv, kMaxGroup, qt));
       names.push_back(decode_sk_name(kv, 3, qt));
-      if (kv != VK_KV_F16) names.push_back(decode_wg_name(kv, 3, qt));
+      names.push_back(decode_wg_name(kv, 3, qt));
       if (kv == VK_KV_F16 || kv == VK_KV_I8_BLK) names.push_back(tree_pfx_name(kv, 3, qt));
       for (int rt : {1, 2}) names.push_back(tree_name(kv, 3, rt, qt));
       names.push_back(decode_mfma_name(kv, 3, qt, true));  // head_dim 64
@@ -322,13 +322,13 @@ extern "C" int vk_ctx_create(int device, const char* code_object_path, vk_ctx** 
     }
   }
   // vk_append_rope_decode's kernels: every kernel that folds the append, suffix _rope
-  for (int kv : {VK_KV_F16, VK_KV_I8_BLK})
+  for (int kv = 0; kv < 4; ++kv)
     for (int g : {1, 2, 4, 8, 3})
       for (int qt : {VK_DT_F16, VK_DT_F32})
         for (bool d64 : {false, true}) {
           if (d64 && g != 3) continue;
-          names.push_back(decode_sk_name(kv, g, qt, d64) + kRopeSuffix);
-          if (kv == VK_KV_I8_BLK) names.push_back(decode_wg_name(kv, g, qt, d64) + kRopeSuffix);
+          if (kv == VK_KV_F16 || kv == VK_KV_I8_BLK) names.push_back(decode_sk_name(kv, g, qt, d64) + kRopeSuffix);
+          names.push_back(decode_wg_name(kv, g, qt, d64) + kRopeSuffix);
         }
   for (int kv = 0; kv < 4; ++kv)
     for (int g : {1, 2, 4, 8}) {
@@ -337,7 +337,7 @@ extern "C" int vk_ctx_create(int device, const char* code_object_path, vk_ctx** 
         names.push_back(decode_mfma_name(kv, g, qt));
         names.push_back(decode_sk_name(kv, g, qt));
         if (kv != VK_KV_F32) names.push_back(decode_pk_name(kv, g, qt));
-        if (kv != VK_KV_F16) names.push_back(decode_wg_name(kv, g, qt));
+        names.push_back(decode_wg_name(kv, g, qt));
       }
       for (int rt : {1, 2})
         for (int qt = 0; qt < 2; ++qt) names.push_back(tree_name(kv, g, rt, qt));
@@ -740,6 +740,23 @@ constexpr int kSkPenalty = 8;
 // workgroup-split decode (vk_append_decode over I8_BLK pools): that wave's range
 // is this much shorter.
 constexpr int kFoldBlocks = 3;
+// Small batches under VK_SCHED_AUTO take the workgroup split in one or a few
+// partitions per sequence (small_plan) while their (sequence, KV head) pairs
+// have at most this many blocks in all: ragged batches; uniform ones; uniform
+// ones over fp16 pools or of at most kFewPairs pairs, where the alternative is
+// split-K of one-wave units.
+constexpr int64_t kSmallRagged = 16384;
+constexpr int64_t kSmallUniform = 12288;
+constexpr int64_t kSmallUniformWide = 65536;
+constexpr int64_t kFewPairs = 64;
+// K and V bytes of the least partition worth a workgroup, and of what a
+// partition must take off the longest context's workgroup to pay for the merge
+// launch it brings (3.4 us; a workgroup alone on its CU streams 43 KB per us).
+constexpr int64_t kMinPartBytes = 65536;
+constexpr int64_t kMergeBytes = 147456;
+// Workgroups of a call in partitions at most: bounds the scratch (17 MB at 16
+// query heads per KV head) and the workgroups past short contexts.
+constexpr int64_t kMaxPartWgs = 2048;
 
 struct DecodePlan {
   const int32_t* bt;
@@ -763,12 +780,15 @@ struct DecodePlan {
 // AUTO (measured faster for each; the VALU kernels compute an fp32 q in fp32
 // and at GQA 8 spill). Over fp16 / int8 KV an fp32 q is split into fp16 hi + lo
 // for the matrix cores; over fp32 KV the matrix cores take q, K, p and V in fp32.
+bool uniform_batch(const vk_decode_args* a) {
+  return a->sum_context_len > 0 &&
+         (double)a->sum_context_len >= 0.97 * (double)a->n_seqs * (double)a->max_context_len;
+}
 void decode_choice(const vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, bool* stream_k, bool* mfma) {
   const vk_pool_desc& d = pool->desc;
   const int kind = ctx ? ctx->decode_kind : VK_DECODE_AUTO;
   const int sched = ctx ? ctx->decode_sched : VK_SCHED_AUTO;
-  const bool uniform = a->sum_context_len > 0 &&
-                       (double)a->sum_context_len >= 0.97 * (double)a->n_seqs * (double)a->max_context_len;
+  const bool uniform = uniform_batch(a);
   const int G = a->n_heads / d.n_kv_heads;
   // the VALU kernels exist for group sizes 1, 2, 4, 8 and head_dim 128 only: the rest always
   // take the matrix cores, and beyond one 16-row tile only fixed partitions
@@ -787,6 +807,45 @@ int auto_partition(const vk_decode_args* a, const vk_pool_desc& d, int64_t resid
   for (int P = 256; P < kMaxPartTokens; P *= 2)
     if (pairs * ((ctx + P - 1) / P) <= resident_waves) return P;
   return kMaxPartTokens;
+}
+
+// Workgroup split of a small batch (VK_SCHED_AUTO): *waves waves per (sequence,
+// partition of *part_blocks blocks, KV head); false when the batch is too large
+// for it. waves_total: resident waves of the kernel; tile: K bytes of one block
+// and KV head. The lengths' sum only steers the choice: any lengths up to
+// max_context_len are computed whatever it says.
+bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves_total, int64_t tile, int* waves,
+                int64_t* part_blocks) {
+  const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
+  const int64_t pairs = (int64_t)a->n_seqs * d.n_kv_heads;
+  if (pairs <= 0 || nb <= 0 || pairs > waves_total) return false;
+  // lengths the host does not know (any up to max_context_len) stay with stream-K,
+  // which balances whatever they are
+  if (a->sum_context_len <= 0 && a->n_seqs > 1) return false;
+  // blocks of one KV head over all sequences (at most, when the lengths are not known)
+  const int64_t most = (int64_t)a->n_seqs * nb;
+  const int64_t sum = a->sum_context_len > 0 ? std::min(most, a->sum_context_len / kBS + a->n_seqs) : most;
+  int64_t limit = kSmallRagged;
+  if (uniform_batch(a)) limit = d.kv_type == VK_KV_F16 || pairs <= kFewPairs ? kSmallUniformWide : kSmallUniform;
+  if (sum * d.n_kv_heads > limit) return false;
+  // uniform contexts of up to four int8 blocks (one fp32 block) take one wave of
+  // split-K, whose result needs no combining (5.6 us per call at two int8 blocks;
+  // fp16 split-K runs the vector kernel, 13.0 us at 16 x 32 tokens against 5.6)
+  if (uniform_batch(a) && d.kv_type != VK_KV_F16 && nb * kv_esz(d.kv_type) <= 4) return false;
+  int nw = nb <= kWgMaxWaves ? kWgMaxWaves / 2 : kWgMaxWaves;
+  while (nw > 1 && pairs * nw > waves_total) nw /= 2;
+  *waves = nw;
+  *part_blocks = nb;
+  if (nw < kWgMaxWaves) return true;
+  // partitions whose workgroups fit one round: at most floor(slots / S) per
+  // sequence, or sum / part + S in all (a partial one per sequence)
+  const int64_t slots = waves_total / kWgMaxWaves / d.n_kv_heads;
+  const int64_t per = std::max<int64_t>(1, slots / a->n_seqs);
+  int64_t part = (nb + per - 1) / per;
+  if (slots > a->n_seqs) part = std::min(part, (sum + slots - a->n_seqs - 1) / (slots - a->n_seqs));
+  part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
+  if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
+  return true;
 }
 
 int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, DecodePlan* pl) {
@@ -822,6 +881,26 @@ int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, Decod
   pl->packed = false;
   pl->max_wave_blocks = 0;
   const int sched = ctx ? ctx->decode_sched : VK_SCHED_AUTO;
+  // (VK_DECODE_VALU asks for the vector kernels of fixed partitions)
+  const bool valu = ctx && ctx->decode_kind == VK_DECODE_VALU && fixed_group(G) && d.head_dim == kHD;
+  int64_t part = 0;
+  int waves = 0;
+  const std::string wg = decode_wg_name(d.kv_type, G, a->q_dtype, d64);
+  if (sched == VK_SCHED_AUTO && !valu && P == 0 && G <= kMaxGroupTile &&
+      small_plan(a, d, ctx ? resident_waves(ctx, wg, 64 * kWgMaxWaves) : 2048, pool->geom.tile_bytes, &waves, &part)) {
+    const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
+    pl->stream_k = false;
+    pl->wg_waves = waves;
+    pl->kernel = wg;
+    pl->part_tokens = (int32_t)part * kBS;
+    pl->max_parts = (int32_t)((nb + part - 1) / part);
+    if (pl->max_parts > 1) {
+      const uint64_t rows = (uint64_t)a->n_seqs * a->n_heads * pl->max_parts;
+      pl->acc_bytes = align_up(rows * kHD * sizeof(float), 256);
+      pl->ml_bytes = align_up(rows * 2 * sizeof(float), 256);
+    }
+    return VK_OK;
+  }
   if (pl->stream_k && sched == VK_SCHED_PACKED && fixed_group(G) && d.kv_type != VK_KV_F32 && a->n_seqs > 0 &&
       a->n_seqs <= kPkMaxSeqs) {
     // Packed workgroup split: one workgroup per resident slot (n_workers bins), the
@@ -940,7 +1019,11 @@ extern "C" int vk_paged_decode_plan(const vk_pool* pool, const vk_decode_args* a
   } else if (pl.wg_waves) {
     out->schedule = VK_SCHED_WORKGROUP;
     out->wg_waves = pl.wg_waves;
-    out->max_blocks_per_wave = (int32_t)((nb + pl.wg_waves - 1) / pl.wg_waves);
+    out->partition_tokens = pl.max_parts > 1 ? pl.part_tokens : 0;
+    out->max_partitions = pl.max_parts > 1 ? pl.max_parts : 0;
+    const int64_t wg_nb = pl.max_parts > 1 ? pl.part_tokens / kBS : nb;
+    out->max_blocks_per_wave = (int32_t)((wg_nb + pl.wg_waves - 1) / pl.wg_waves);
+    out->merge_launch = pl.max_parts > 1 ? 1 : 0;
   } else {
     out->schedule = VK_SCHED_SPLIT;
     out->partition_tokens = pl.part_tokens;
@@ -958,10 +1041,15 @@ namespace {
 // slots derived in the kernel (the unfused half of vk_append_decode).
 // Whether the decode launch of this plan appends the new tokens itself
 // (vk_append_decode): I8_BLK pools under the workgroup split or stream-K, fp16
-// pools under stream-K, over tiles the folded kernels are built for.
+// pools for ragged batches under either, and any pool for one sequence under the
+// workgroup split, over tiles the folded kernels are built for. Several sequences
+// of the other types keep the append launch: the call may list one sequence at
+// two lengths, and the longer row must see the shorter one's token.
 bool plan_folds_append(const vk_pool* pool, const vk_decode_args* a, const DecodePlan& pl) {
   const int kvt = pool->desc.kv_type;
-  return ((kvt == VK_KV_I8_BLK && (pl.wg_waves > 0 || pl.stream_k)) || (kvt == VK_KV_F16 && pl.stream_k)) &&
+  const bool alone = a->n_seqs == 1 && pl.wg_waves > 0;
+  return ((kvt == VK_KV_I8_BLK && (pl.wg_waves > 0 || pl.stream_k)) ||
+          (kvt == VK_KV_F16 && (pl.stream_k || (pl.wg_waves > 0 && !uniform_batch(a)))) || alone) &&
          (tile_hd(pool->desc.head_dim) == kHD || use_d64(pool->desc, a->n_heads / pool->desc.n_kv_heads));
 }
 
@@ -1031,10 +1119,9 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
   if (a->n_seqs == 0) return VK_OK;
   if (!a->q || !a->out || !a->context_lens) return fail(VK_ERR_BAD_ARG, "null device pointer");
   if ((rc = set_device(ctx))) return rc;
-  // I8_BLK pools under the workgroup split or stream-K, and fp16 pools under
-  // stream-K, take the append inside the decode launch (the wave that holds a
-  // sequence's last block appends the token before loading it); every other
-  // plan appends in a launch of its own first
+  // plan_folds_append: the append inside the decode launch (the wave that holds a
+  // sequence's last block appends the token before loading it); every other plan
+  // appends in a launch of its own first
   const int kvt = pool->desc.kv_type;
   const bool fold = k_new && plan_folds_append(pool, a, pl);
   const bool rope_fold = fold && rope.style != ROPE_NONE && plan_folds_rope(pool, a, pl);
@@ -1107,7 +1194,7 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
     // workgroup split: the folding wave's range is shortened by kFoldBlocks
     // while every wave's share stays within its four block-id windows (stream-K
     // ranges are not shortened)
-    const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
+    const int64_t nb = pl.max_parts > 1 ? pl.part_tokens / kBS : ((int64_t)a->max_context_len + kBS - 1) / kBS;
     p.fold_blocks = pl.wg_waves > 0 && (nb + kFoldBlocks + pl.wg_waves - 1) / pl.wg_waves <= kMaxPartTokens / kBS
                         ? kFoldBlocks : 0;
   }
@@ -1139,9 +1226,12 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
   }
   if (pl.packed)
     return launch(ctx, kernel.c_str(), dim3((unsigned)pl.n_workers), dim3(64 * kWgMaxWaves), p, stream);
-  if (pl.wg_waves)
-    return launch(ctx, kernel.c_str(), dim3((unsigned)(a->n_seqs * d.n_kv_heads)), dim3(64 * (unsigned)pl.wg_waves),
-                  p, stream);
+  if (pl.wg_waves) {
+    if ((rc = launch(ctx, kernel.c_str(), dim3((unsigned)(a->n_seqs * pl.max_parts * d.n_kv_heads)),
+                     dim3(64 * (unsigned)pl.wg_waves), p, stream)))
+      return rc;
+    return pl.max_parts > 1 ? launch(ctx, "vk_decode_merge", merge_grid, dim3(256), m, stream) : VK_OK;
+  }
   const uint64_t units = (uint64_t)a->n_seqs * pl.max_parts * d.n_kv_heads;
   if (units > 0x7FFFFFFFull) return fail(VK_ERR_UNSUPPORTED, "grid too large");
   if ((rc = launch(ctx, kernel.c_str(), dim3((unsigned)units), dim3(64), p, stream))) return rc;

@@ -1177,6 +1177,23 @@ DEV void fold_claim_check(const FoldIn& f, const DecodeParams& P, int s) {
   }
 }
 
+// New row e (0 K, 1 V) of an I8_REF pool by append_ref's rule: fp32 scale
+// amax / 127, codes trunc(x * (127 / amax)).
+template <bool IS_V, int D>
+DEV void fold_ref_row(const FoldIn& f, const DecodeParams& P) {
+  const int lane = lane_id();
+  const float x0 = f.x[IS_V][0], x1 = f.x[IS_V][1];
+  const float amax = wave_max(fmaxf(fabsf(x0), fabsf(x1)));
+  const float inv = amax > 0.f ? 127.0f / amax : 0.f;
+  uint8_t* tile = const_cast<uint8_t*>(IS_V ? P.vc : P.kc) + f.tix * P.tile_bytes;
+  if (2 * lane < D) {
+    tile[tile_elem<IS_V>(f.o, 2 * lane, 1, D)] = (uint8_t)(int8_t)(int)(x0 * inv);
+    tile[tile_elem<IS_V>(f.o, 2 * lane + 1, 1, D)] = (uint8_t)(int8_t)(int)(x1 * inv);
+  }
+  if (lane == 0)
+    reinterpret_cast<float*>(const_cast<uint8_t*>(IS_V ? P.vs : P.ks))[f.tix * BS + f.o] = amax / 127.0f;
+}
+
 // The rule, the stores, and the block's new scales in bw.
 template <int KV, int D, bool ROPE = false>
 DEV void fold_finish(FoldIn& f, const DecodeParams& P, BlockIds& bw, int nblk, int s) {
@@ -1207,6 +1224,20 @@ DEV void fold_finish(FoldIn& f, const DecodeParams& P, BlockIds& bw, int nblk, i
       *reinterpret_cast<uint16_t*>(vt + tile_elem<true>(f.o, d0, 2, D)) = f2h(f.x[1][0]);
       *reinterpret_cast<uint16_t*>(vt + tile_elem<true>(f.o, d0 + 1, 2, D)) = f2h(f.x[1][1]);
     }
+    return;
+  } else if constexpr (KV == KV_F32) {  // the new rows as they are, as vk_append_kv0 stores them
+    const int d0 = 2 * lane;
+    if (d0 < D) {
+      uint8_t* kt = const_cast<uint8_t*>(P.kc) + f.tix * P.tile_bytes;
+      uint8_t* vt = const_cast<uint8_t*>(P.vc) + f.tix * P.tile_bytes;
+      *reinterpret_cast<float2*>(kt + tile_elem<false>(f.o, d0, 4, D)) = make_float2(f.x[0][0], f.x[0][1]);
+      *reinterpret_cast<float*>(vt + tile_elem<true>(f.o, d0, 4, D)) = f.x[1][0];
+      *reinterpret_cast<float*>(vt + tile_elem<true>(f.o, d0 + 1, 4, D)) = f.x[1][1];
+    }
+    return;
+  } else if constexpr (KV == KV_I8_REF) {
+    fold_ref_row<false, D>(f, P);
+    fold_ref_row<true, D>(f, P);
     return;
   }
   const uint32_t ks = fold_finish_one<false, D>(f, P);
@@ -1277,7 +1308,7 @@ DEV void attn_piece(const DecodeParams& P, int s, int kvh, int rg, int start, in
   // vk_append_decode with the append folded in: this piece holds the last token
   // and appends it (after the first stage's loads and q, unless the block is in
   // the first stage)
-  static_assert(!FOLD || ((BLK || KV == KV_F16) && !TREE), "the folded append is the I8_BLK and fp16 decode's");
+  static_assert(!FOLD || !TREE, "the folded append is the decode's");
   static_assert(!ROPE || FOLD, "RoPE folds with the folded append");
   // vk_append_decode with the append folded in: this piece holds the last token.
   // Its block in the first stage: append before any tile load; otherwise issue
@@ -1715,7 +1746,39 @@ DEV void f32_stage_load(F32Stage<DF>& st, const DecodeParams& P, const BlockIds&
       st.v[t][r] = __builtin_amdgcn_raw_buffer_load_b64(vr, (t < 4 ? v0 : v1) + 128 * t, r * 8 * D, kAuxNT);
 }
 
-template <int G, int RT, bool TREE, int QT, int DF = HD>
+// RoPE of the piece's q rows (vk_append_rope_decode) at table row csr: the lane
+// holds dims 16 j + 4 g + e, so the partner of a value (e ^ 1 interleaved, NJ / 2
+// chunks away half-split) is its own. t: the lane's (cos, sin) pairs, chunk j's
+// two (interleaved) or those of chunks j and j + NJ / 2 (half-split, entries
+// 2 j and 2 j + 1, j < NJ / 2). rope_rotate's expressions and order, both styles
+// in one branch-free form as in rope_q_finish.
+template <int NJ>
+DEV void rope_q_f32_issue(float4 (&t)[NJ], const float* csr, bool half, int g) {
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    t[j] = *reinterpret_cast<const float4*>(csr + (half ? 32 * (j >> 1) + 8 * g + 4 * (j & 1) : 16 * j + 4 * g));
+}
+template <int NJ>
+DEV void rope_q_f32_finish(float (&q)[4 * NJ], const float4 (&t)[NJ], bool half) {
+#pragma clang fp contract(off)
+  float y[4 * NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int jp = (j + NJ / 2) % NJ;                       // half-split partner chunk
+      const float4 ti = t[j], th = t[2 * (j % (NJ / 2)) + (e >> 1)];
+      const float c = half ? ((e & 1) ? th.z : th.x) : ((e >> 1) ? ti.z : ti.x);
+      const float sn = half ? ((e & 1) ? th.w : th.y) : ((e >> 1) ? ti.w : ti.y);
+      const float x = q[4 * j + e], p = half ? q[4 * jp + e] : q[4 * j + (e ^ 1)];
+      const bool first = half ? j < NJ / 2 : (e & 1) == 0;
+      y[4 * j + e] = first ? x * c - p * sn : p * sn + x * c;
+    }
+#pragma unroll
+  for (int i = 0; i < 4 * NJ; ++i) q[i] = y[i];
+}
+
+template <int G, int RT, bool TREE, int QT, int DF = HD, bool FOLD = false, bool ROPE = false>
 DEV void attn_piece_f32(const DecodeParams& P, int s, int kvh, int rg, int start, int end, int ctx_c, bool direct,
                         int64_t pbase, int pstride, float* pacc, float* pml) {
   constexpr int NJ = DF / 16;  // 16-dim groups: score chunks of 4 instructions, value tiles
@@ -1736,6 +1799,23 @@ DEV void attn_piece_f32(const DecodeParams& P, int s, int kvh, int rg, int start
 
   BlockIds bw;
   load_block_ids<false>(bw, P, bt, blk0, nblk, kvh);
+  // the folded append and RoPE, as in attn_piece
+  static_assert(!FOLD || !TREE, "the folded append is the decode's");
+  static_assert(!ROPE || (FOLD && RT == 1), "RoPE folds with the folded append");
+  bool fold = false;
+  if constexpr (FOLD) fold = P.fold_k != nullptr && end == ctx_c && nblk > 0;
+  const bool fold_first = fold && nblk <= 1;
+  FoldIn fin;
+  if constexpr (FOLD) {
+    if (fold) fold_issue<KV_F32, DF, ROPE>(fin, P, bw, nblk, s, kvh, ctx_c);
+    if (fold_first) fold_finish<KV_F32, DF, ROPE>(fin, P, bw, nblk, s);
+  }
+  float4 rt4[ROPE ? NJ : 1];
+  bool rot = false;
+  if constexpr (ROPE) {
+    rot = ctx_c - 1 >= 0 && ctx_c - 1 < P.rope_n_pos;
+    rope_q_f32_issue<NJ>(rt4, P.cos_sin + (int64_t)(rot ? ctx_c - 1 : 0) * P.io_hd, P.rope == ROPE_HALF, g);
+  }
   F32Stage<DF> sa, sb;
   f32_stage_load<DF>(sa, P, bw, 0, nblk, kvh, n, g);
 
@@ -1759,10 +1839,21 @@ DEV void attn_piece_f32(const DecodeParams& P, int s, int kvh, int rg, int start
       }
       qf[rt][4 * j] = x.x; qf[rt][4 * j + 1] = x.y; qf[rt][4 * j + 2] = x.z; qf[rt][4 * j + 3] = x.w;
     }
+    if constexpr (ROPE) {
+      if (rot) rope_q_f32_finish<NJ>(qf[rt], rt4, P.rope == ROPE_HALF);
+      if constexpr (QT == DT_F16) {  // the RoPE append stores a rotated fp16 q rounded to fp16
+#pragma unroll
+        for (int i = 0; i < 4 * NJ; ++i) qf[rt][i] = rot ? (float)(_Float16)qf[rt][i] : qf[rt][i];
+      }
+    }
     mrow[rt] = 0u;
     if constexpr (TREE) {
       if (R < nrows) mrow[rt] = P.tree_mask[(int64_t)s * N + R / Gn];
     }
+  }
+
+  if constexpr (FOLD) {
+    if (fold && !fold_first) fold_finish<KV_F32, DF, ROPE>(fin, P, bw, nblk, s);
   }
 
   float M[RT], lrun[RT];
@@ -1896,7 +1987,7 @@ template <int KV, int G, int RT, bool TREE, int QT, int D = HD, bool FOLD = fals
 DEV void attn_piece_kv(const DecodeParams& P, int s, int kvh, int rg, int start, int end, int ctx_c, bool direct,
                        int64_t pbase, int pstride, float* pacc, float* pml, int npre = 0) {
   if constexpr (KV == KV_F32) {
-    attn_piece_f32<G, RT, TREE, QT, D>(P, s, kvh, rg, start, end, ctx_c, direct, pbase, pstride, pacc, pml);
+    attn_piece_f32<G, RT, TREE, QT, D, FOLD, ROPE>(P, s, kvh, rg, start, end, ctx_c, direct, pbase, pstride, pacc, pml);
   } else {
     attn_piece<KV, G, RT, TREE, QT, D, FOLD, ROPE>(P, s, kvh, rg, start, end, ctx_c, direct, pbase, pstride, pacc, pml, npre);
   }
@@ -1965,13 +2056,15 @@ DEV int wave_sum_i(int x) {
   x += __shfl_xor(x, 32, WAVE);
   return x;
 }
+// Inclusive scan over the wave on the VALU: row shifts, then lane 15 of rows 0
+// and 2 to the row after each, then lane 31 to the upper half.
 DEV int wave_incl_scan_i(int x) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int d = 1; d < WAVE; d <<= 1) {
-    const int y = __shfl_up(x, d, WAVE);
-    if (lane >= d) x += y;
-  }
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast 15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast 31
   return x;
 }
 DEV int seq_blocks(const DecodeParams& P, int s) {
@@ -2056,13 +2149,45 @@ DEV void attn_streamk_mfma(const DecodeParams& P) {
 }
 
 // ---- workgroup-split decode ------------------------------------------------
-// One workgroup of NW = blockDim.x / 64 waves per (sequence, KV head), KV head
-// fastest: wave w takes the w-th of NW equal block ranges of the context,
-// leaves its unnormalised partial (acc, M, l) in LDS, and after one barrier the
-// workgroup combines them into the output rows,
-//   out = sum_w 2^(M_w - M) acc_w / sum_w 2^(M_w - M) l_w,  M = max_w M_w,
-// so a uniform batch needs no partials in HBM and no merge launch.
+// One workgroup of NW = blockDim.x / 64 waves per (sequence, partition of
+// part_tokens tokens, KV head), KV head fastest: wave w takes the w-th of NW
+// equal block ranges of the partition, leaves its unnormalised partial (acc, M,
+// l) in LDS, and after one barrier the workgroup combines them,
+//   out = sum_w 2^(M_w - M) acc_w / sum_w 2^(M_w - M) l_w,  M = max_w M_w.
+// A context of one partition is written as output rows: no partials in HBM and
+// no merge launch (uniform batches that fill the GPU, and short contexts). A
+// longer one leaves one partial per partition for vk_decode_merge; combining
+// the waves first keeps that merge to an eighth of the partials that one-wave
+// units would leave.
 constexpr int kWgMaxWaves = 8;
+// Partition i of the batch, the sequences' partitions in order (an empty context
+// has one, which writes its zero rows): its sequence s and place in it; false
+// past the last. Numbering only the partitions that exist spreads the work
+// evenly over the XCDs, which take consecutive workgroups in turn, and leaves
+// the grid's surplus (it is sized for max_context_len) at its end; a grid of
+// max_parts per sequence gave some XCDs two rounds of full partitions and others
+// mostly workgroups past short contexts (16 ragged contexts of up to 2048
+// tokens over int8: 25.2 us per call against 18.3).
+DEV bool wg_part_of(const DecodeParams& P, int i, int& s, int& part) {
+  const int lane = lane_id();
+  int off = 0;
+  for (int b = 0; b < P.n_seqs; b += WAVE) {
+    const int sl = b + lane;
+    const int ctx = sl < P.n_seqs ? max(1, min(P.context_lens[sl], P.cap_tokens)) : 0;
+    const int np = (ctx + P.part_tokens - 1) / P.part_tokens;
+    const int incl = wave_incl_scan_i(np);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(off + incl > i);
+    if (m != 0) {
+      const int l = __builtin_ctzll(m);
+      s = b + l;
+      part = i - off - readlane_i(incl - np, l);
+      return true;
+    }
+    off += readlane_i(incl, WAVE - 1);
+  }
+  return false;
+}
+
 template <int KV, int G, int QT = DT_F16, int D = HD, bool ROPE = false>
 DEV void attn_wg_mfma(const DecodeParams& P) {
   constexpr int GM = lds_rows<G>();
@@ -2073,43 +2198,68 @@ DEV void attn_wg_mfma(const DecodeParams& P) {
   const int w = (int)threadIdx.x / WAVE;
   const int lane = lane_id();
   const int kvh = (int)blockIdx.x % P.n_kv_heads;
-  const int s = (int)blockIdx.x / P.n_kv_heads;
-  if (s >= P.n_seqs) return;  // the whole workgroup
+  int s = (int)blockIdx.x / P.n_kv_heads, part = 0;
+  if (P.max_parts > 1) {
+    if (!wg_part_of(P, s, s, part)) return;  // the whole workgroup
+  } else if (s >= P.n_seqs) {
+    return;
+  }
   const int ctx = max(0, min(P.context_lens[s], P.cap_tokens));
   if (ctx == 0) {
     if (w == 0) write_zero_rows_n(P, s, kvh, Gn);
     return;
   }
-  const int nb = (ctx + BS - 1) / BS;
-  // under vk_append_decode (I8_BLK) the wave whose range ends at the context's
-  // last token appends the new token first (fold_issue, fold_finish): the split
-  // counts that append as fold_blocks more blocks of that wave's range
-  const int fw = (KV == KV_I8_BLK && P.fold_k != nullptr) ? P.fold_blocks : 0;
+  // blocks [pb, pe) of the context are this partition's
+  const int nb_ctx = (ctx + BS - 1) / BS, pblk = P.part_tokens / BS;
+  const int pb = P.max_parts > 1 ? part * pblk : 0;
+  const int pe = P.max_parts > 1 ? min(nb_ctx, pb + pblk) : nb_ctx;
+  const int nb = pe - pb;
+  // under vk_append_decode the wave whose range ends at the context's last token
+  // appends the new token first (fold_issue, fold_finish): the split counts that
+  // append as fold_blocks more blocks of that wave's range
+  const int fw = P.fold_k != nullptr && pe == nb_ctx ? P.fold_blocks : 0;
   const int per = (nb + fw + nw - 1) / nw;
   const int b0 = min(nb, w * per), b1 = min(nb, b0 + per);
   if (b0 < b1) {
-    attn_piece_kv<KV, G, 1, false, QT, D, KV == KV_I8_BLK, ROPE>(P, s, kvh, 0, b0 * BS, min(b1 * BS, ctx), ctx, false, 0, 1,
-                                                           &wacc[w][0][0], &wml[w][0][0]);
+    attn_piece_kv<KV, G, 1, false, QT, D, true, ROPE>(P, s, kvh, 0, (pb + b0) * BS, min((pb + b1) * BS, ctx), ctx,
+                                                      false, 0, 1, &wacc[w][0][0], &wml[w][0][0]);
   } else if (lane < Gn) {
     wml[w][lane][0] = kNegInf;
     wml[w][lane][1] = 0.f;
   }
   __syncthreads();
+  const bool whole = nb == nb_ctx;
   const int64_t hrow0 = (int64_t)s * P.n_heads + (int64_t)kvh * Gn;
   const int IO = P.io_hd;  // output dims of a row; the partials are HD wide
-  for (int i = (int)threadIdx.x; i < Gn * IO; i += (int)blockDim.x) {
-    const int r = i / IO, d = i - r * IO;
-    float M = kNegInf;
-    for (int v = 0; v < nw; ++v) M = fmaxf(M, wml[v][r][0]);
-    float L = 0.f, o = 0.f;
-    for (int v = 0; v < nw; ++v) {
-      const float mv = wml[v][r][0];
-      if (mv == kNegInf) continue;  // a wave with no tokens (its acc row is not written)
-      const float e = __builtin_amdgcn_exp2f(mv - M);
-      L = fmaf(e, wml[v][r][1], L);
-      o = fmaf(e, wacc[v][r][d], o);
+  for (int e = (int)threadIdx.x; e < Gn * IO; e += (int)blockDim.x) {
+    const int r = IO == HD ? e / HD : e / IO, d = e - r * IO;
+    // every wave's values read at once (the LDS rows of waves past nw, and the
+    // acc rows of waves with no tokens, hold anything: selected away)
+    float m[kWgMaxWaves], l[kWgMaxWaves], a[kWgMaxWaves];
+#pragma unroll
+    for (int v = 0; v < kWgMaxWaves; ++v) {
+      const float2 ml = *reinterpret_cast<const float2*>(&wml[v][r][0]);
+      m[v] = v < nw ? ml.x : kNegInf;
+      l[v] = ml.y;
+      a[v] = wacc[v][r][d];
     }
-    P.out[(hrow0 + r) * IO + d] = L > 0.f ? o / L : 0.f;
+    float M = kNegInf;
+#pragma unroll
+    for (int v = 0; v < kWgMaxWaves; ++v) M = fmaxf(M, m[v]);
+    float L = 0.f, o = 0.f;
+#pragma unroll
+    for (int v = 0; v < kWgMaxWaves; ++v) {
+      const float ev = m[v] == kNegInf ? 0.f : __builtin_amdgcn_exp2f(m[v] - M);
+      L = m[v] == kNegInf ? L : fmaf(ev, l[v], L);
+      o = m[v] == kNegInf ? o : fmaf(ev, a[v], o);
+    }
+    if (whole) {
+      P.out[(hrow0 + r) * IO + d] = L > 0.f ? o / L : 0.f;
+    } else {
+      const int64_t pr = (hrow0 + r) * P.max_parts + part;
+      P.part_acc[pr * HD + d] = o;
+      if (d == 0) reinterpret_cast<float2*>(P.part_ml)[pr] = make_float2(M, L);
+    }
   }
 }
 
@@ -2641,29 +2791,36 @@ DEV void tree_prefix_mfma(const DecodeParams& P) {
 // One wave per (sequence, head); sequences with a single partition were
 // finished by the decode kernel itself. Partial rows are loaded 8 at a time so
 // the loads overlap.
-// Combine np partials (index pr(k), k = 0..np-1) into one output row.
+// Combine np partials (index pr(k), k = 0..np-1) into one output row. m0, a0: the
+// (M, l) pair of partial `lane` and the lane's dims of partials 0..7, loaded by
+// the caller (any value where there is no such partial).
 template <typename PR>
-DEV void merge_row(const MergeParams& P, int64_t out_row, int np, PR pr) {
+DEV void merge_row(const MergeParams& P, int64_t out_row, int np, PR pr, float2 m0, const float2 (&a0)[8]) {
   const int lane = lane_id();
   const float2* ml = reinterpret_cast<const float2*>(P.part_ml);
   const float2* pa = reinterpret_cast<const float2*>(P.part_acc);
-  float M = kNegInf;
-  for (int p = lane; p < np; p += WAVE) M = fmaxf(M, ml[pr(p)].x);
+  float M = lane < np ? m0.x : kNegInf;
+  for (int p = lane + WAVE; p < np; p += WAVE) M = fmaxf(M, ml[pr(p)].x);
   M = wave_max(M);
   float L = 0.f, o0 = 0.f, o1 = 0.f;
   for (int p0 = 0; p0 < np; p0 += WAVE) {
     float w = 0.f;
     if (p0 + lane < np) {
-      const float2 m = ml[pr(p0 + lane)];
+      const float2 m = p0 == 0 ? m0 : ml[pr(p0 + lane)];
       w = (m.x == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m.x - M);
       L = fmaf(w, m.y, L);
     }
     const int cnt = min(WAVE, np - p0);
     for (int k0 = 0; k0 < cnt; k0 += 8) {
       float2 a[8];
+      if (p0 == 0 && k0 == 0) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        a[k] = (k0 + k < cnt) ? pa[pr(p0 + k0 + k) * (HD / 2) + lane] : make_float2(0.f, 0.f);
+        for (int k = 0; k < 8; ++k) a[k] = a0[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          a[k] = (k0 + k < cnt) ? pa[pr(p0 + k0 + k) * (HD / 2) + lane] : make_float2(0.f, 0.f);
+      }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const float wk = readlane_f(w, min(k0 + k, cnt - 1));
@@ -2679,6 +2836,16 @@ DEV void merge_row(const MergeParams& P, int64_t out_row, int np, PR pr) {
   if (2 * lane < P.io_hd)
     reinterpret_cast<float2*>(P.out)[out_row * (P.io_hd / 2) + lane] = make_float2(o0 * inv, o1 * inv);
 }
+// The loads of merge_row's first partials (np of them, or at most: indices past
+// the last read the last).
+template <typename PR>
+DEV void merge_first(const MergeParams& P, int np, PR pr, float2& m0, float2 (&a0)[8]) {
+  const int lane = lane_id(), last = max(np - 1, 0);
+  m0 = reinterpret_cast<const float2*>(P.part_ml)[pr(min(lane, last))];
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    a0[k] = reinterpret_cast<const float2*>(P.part_acc)[pr(min(k, last)) * (HD / 2) + lane];
+}
 
 // Split-K merge: one wave per (sequence, row) with partials [row][max_parts]:
 //   out = sum_p 2^(M_p - M) acc_p / sum_p 2^(M_p - M) l_p,  M = max_p M_p.
@@ -2686,18 +2853,24 @@ DEV void merge_row(const MergeParams& P, int64_t out_row, int np, PR pr) {
 // With a shared prefix (tree verify), slots 0..prefix_chunks-1 hold the prefix
 // pass and the partitions of the rest follow; a row whose rest fits one
 // partition was finished by the tree kernel (it folds the prefix slots in).
+// The first partials are loaded beside the context length (from slots that
+// exist, used only if the row has them): one round trip where a short merge had
+// three.
 __device__ void decode_merge(const MergeParams& P) {
   const int r = blockIdx.x * (blockDim.x / WAVE) + (threadIdx.x / WAVE);
   if (r >= P.n_rows) return;
   const int s = r / P.rows_per_seq;
+  const int64_t base = (int64_t)r * P.max_parts;
+  const auto pr = [=](int k) -> int64_t { return base + k; };
+  float2 m0, a0[8];
+  merge_first(P, P.max_parts, pr, m0, a0);
   const int ctx_c = max(0, min(P.context_lens[s], P.cap_tokens));
   const int ctx = min(ctx_c + P.extra_tokens, P.cap_tokens);
   const int pre = P.prefix_chunks > 0 ? prefix_tokens_of(ctx_c, P.prefix_blocks) : 0;
   const int np = P.prefix_chunks + (ctx - pre + P.part_tokens - 1) / P.part_tokens;
   // one partition, or one after the prefix chunks: the attention kernel wrote the row
   if (np == P.prefix_chunks + 1) return;
-  const int64_t base = (int64_t)r * P.max_parts;
-  merge_row(P, r, np, [&](int k) -> int64_t { return base + k; });
+  merge_row(P, r, np, pr, m0, a0);
 }
 
 // Stream-K merge: one wave per (sequence, head). The segment (s, kvh) starts at
@@ -2723,9 +2896,11 @@ __device__ void decode_merge_sk(const MergeParams& P) {
   int w_lo, w_hi;
   sk_segment_workers(sp, seg0, nb, P.sk_penalty, &w_lo, &w_hi);
   if (w_lo == w_hi) return;
-  merge_row(P, r, w_hi - w_lo + 1, [&](int k) -> int64_t {
-    return ((int64_t)(w_lo + k) * 2 + (k == 0 ? 1 : 0)) * G + gi;
-  });
+  const int wl = w_lo, np = w_hi - w_lo + 1;
+  const auto pr = [=](int k) -> int64_t { return ((int64_t)(wl + k) * 2 + (k == 0 ? 1 : 0)) * G + gi; };
+  float2 m0, a0[8];
+  merge_first(P, np, pr, m0, a0);
+  merge_row(P, r, np, pr, m0, a0);
 }
 
 // =============================================================================
@@ -3478,14 +3653,14 @@ VK_DECODE_MFMA_Q0_G(0) VK_DECODE_MFMA_Q0_G(1) VK_DECODE_MFMA_Q0_G(2) VK_DECODE_M
     attn_wg_mfma<KV, G>(P);                                                         \
   }
 #define VK_DECODE_WG_G(KV) VK_DECODE_WG(KV, 1) VK_DECODE_WG(KV, 2) VK_DECODE_WG(KV, 4) VK_DECODE_WG(KV, 8)
-VK_DECODE_WG_G(0) VK_DECODE_WG_G(2) VK_DECODE_WG_G(3)
+VK_DECODE_WG_G(0) VK_DECODE_WG_G(1) VK_DECODE_WG_G(2) VK_DECODE_WG_G(3)
 #define VK_DECODE_WG_Q0(KV, G)                                                      \
   extern "C" __global__ void __launch_bounds__(64 * kWgMaxWaves)                    \
       vk_decode_wg_kv##KV##_g##G##_q0(const DecodeParams P) {                       \
     attn_wg_mfma<KV, G, DT_F32>(P);                                                 \
   }
 #define VK_DECODE_WG_Q0_G(KV) VK_DECODE_WG_Q0(KV, 1) VK_DECODE_WG_Q0(KV, 2) VK_DECODE_WG_Q0(KV, 4) VK_DECODE_WG_Q0(KV, 8)
-VK_DECODE_WG_Q0_G(0) VK_DECODE_WG_Q0_G(2) VK_DECODE_WG_Q0_G(3)
+VK_DECODE_WG_Q0_G(0) VK_DECODE_WG_Q0_G(1) VK_DECODE_WG_Q0_G(2) VK_DECODE_WG_Q0_G(3)
 
 // Packed workgroup split (ragged batches): up to kWgMaxWaves waves of 64.
 #define VK_DECODE_PK(KV, G, QT, SUF)                                                \
@@ -3562,7 +3737,7 @@ VK_GX_DECODE(0) VK_GX_DECODE(1) VK_GX_DECODE(2) VK_GX_DECODE(3)
   extern "C" __global__ void __launch_bounds__(64 * kWgMaxWaves) vk_decode_wg_kv##KV##_gx_q0(const DecodeParams P) { \
     attn_wg_mfma<KV, 0, DT_F32>(P);                                                                            \
   }
-VK_GX_WG(0) VK_GX_WG(2) VK_GX_WG(3)
+VK_GX_WG(0) VK_GX_WG(1) VK_GX_WG(2) VK_GX_WG(3)
 // head_dim 64 (64-dim pieces, any group size up to 16): split-K, stream-K and
 // the workgroup split
 #define VK_D64_DECODE(KV)                                                                                       \
@@ -3617,7 +3792,8 @@ VK_D64_WG(0) VK_D64_WG(1) VK_D64_WG(2) VK_D64_WG(3)
   M(KV, _gx, DT_F16, HD) M(KV, _gx_d64, DT_F16, HD / 2)                                          \
   M(KV, _g1_q0, DT_F32, HD) M(KV, _g2_q0, DT_F32, HD) M(KV, _g4_q0, DT_F32, HD)                  \
   M(KV, _g8_q0, DT_F32, HD) M(KV, _gx_q0, DT_F32, HD) M(KV, _gx_d64_q0, DT_F32, HD / 2)
-VK_ROPE_ALL(VK_ROPE_SK, 1) VK_ROPE_ALL(VK_ROPE_SK, 3) VK_ROPE_ALL(VK_ROPE_WG, 3)
+VK_ROPE_ALL(VK_ROPE_SK, 1) VK_ROPE_ALL(VK_ROPE_SK, 3)
+VK_ROPE_ALL(VK_ROPE_WG, 0) VK_ROPE_ALL(VK_ROPE_WG, 1) VK_ROPE_ALL(VK_ROPE_WG, 2) VK_ROPE_ALL(VK_ROPE_WG, 3)
 #define VK_GX_TREE(KV, RT, QT, ATTR)                                                                            \
   extern "C" __global__ void __launch_bounds__(64) ATTR vk_tree_kv##KV##_gx_r##RT##_q##QT(const DecodeParams P) { \
     attn_unit_mfma<KV, 0, RT, true, QT>(P);                                                                    \
