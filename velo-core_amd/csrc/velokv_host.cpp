@@ -596,12 +596,41 @@ extern "C" int vk_slot_mapping(vk_ctx* ctx, vk_pool* pool, const int32_t* block_
 }
 
 namespace {
-// Tokens per append workgroup: enough workgroups to spread the runs over the GPU
-// (about 2048 per call), at most 64 (one slot load per lane); a workgroup per
-// token for small calls.
+// Tokens per workgroup of the I8_BLK runs: about 2048 workgroups per call, one
+// token each for small calls, and at most a block's 16 (a prompt's blocks then
+// have a workgroup each; 64 left 1,000 workgroups with four runs in turn at
+// 8,000 tokens x 8 heads).
 int append_tok_per_wg(int32_t n_tok, int32_t n_kv_heads) {
   const int64_t t = ((int64_t)n_tok * n_kv_heads + 2047) / 2048;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(64, t));
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kBS, t));
+}
+
+// Appends of the other types up to this many (token, KV head) pairs have a workgroup
+// for each, all of them resident at once; longer ones take rows four tokens a wave.
+// 624 pairs: 3.5 us against 4.0 in the kernel; 2,048 pairs with 32 query heads level
+// (5.5 us each, int8 5.4 and 5.9); 6,216 pairs: 12.6 us against 6.0.
+constexpr int64_t kTokenWgs = 2048;
+
+// Launches an append (AppendParams filled but for its grid).
+int launch_append(const vk_ctx* ctx, const vk_pool* pool, AppendParams& p, void* stream) {
+  constexpr int kRowTokens = 8;  // velokv_kernels.hip
+  const int hkv = pool->desc.n_kv_heads;
+  const bool blk = pool->desc.kv_type == VK_KV_I8_BLK;
+  p.tok_per_wg = append_tok_per_wg(p.n_tok, hkv);
+  const auto* none = reinterpret_cast<const int32_t*>(ctx->err_word);
+  p.slot_any = p.slot_mapping ? p.slot_mapping : reinterpret_cast<const int64_t*>(none);
+  p.pos_any = p.positions ? p.positions : none;
+  p.ctx_any = p.slot_mapping ? none : p.context_lens;
+  const int rb = row_batch(pool->desc.kv_type);
+  const bool by_token = (int64_t)p.n_tok * hkv <= kTokenWgs;
+  p.row_groups = (p.n_heads + rb - 1) / rb + (blk || by_token ? 0 : 2 * hkv);
+  const int64_t runs = blk ? ((int64_t)p.n_tok + p.tok_per_wg - 1) / p.tok_per_wg * hkv
+                           : by_token ? (int64_t)p.n_tok * hkv : 0;
+  const int64_t rows = ((int64_t)p.n_tok + kRowTokens - 1) / kRowTokens * p.row_groups;
+  if (runs + rows > 0x7FFFFFFF) return fail(VK_ERR_UNSUPPORTED, "grid too large");
+  p.kv_wgs = (int32_t)runs;
+  const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
+  return launch(ctx, name.c_str(), dim3((unsigned)(runs + rows)), dim3(128), p, stream);
 }
 }  // namespace
 
@@ -623,14 +652,11 @@ extern "C" int vk_append(vk_ctx* ctx, vk_pool* pool, int32_t layer, const void* 
   p.v = v;
   p.slot_mapping = slot_mapping;
   p.n_tok = n_tok;
-  p.tok_per_wg = append_tok_per_wg(n_tok, pool->desc.n_kv_heads);
   p.err = ctx->err_word;
   p.claim = pool->claim;
   p.epoch = pool->claim ? pool->next_epoch() : 0u;
-  const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
   if ((rc = set_device(ctx))) return rc;
-  return launch(ctx, name.c_str(), dim3((unsigned)((n_tok + p.tok_per_wg - 1) / p.tok_per_wg),
-                                        (unsigned)pool->desc.n_kv_heads), dim3(128), p, stream);
+  return launch_append(ctx, pool, p, stream);
 }
 
 extern "C" int vk_rope_table(float* out, int32_t n_pos, int32_t head_dim, float freq_base) {
@@ -680,15 +706,11 @@ extern "C" int vk_append_rope(vk_ctx* ctx, vk_pool* pool, int32_t layer, void* q
   p.n_heads = q ? n_heads : 0;
   p.q = q;
   p.q_dtype = q_dtype;
-  const unsigned rows = (unsigned)pool->desc.n_kv_heads + (q ? (unsigned)((n_heads + 1) / 2) : 0u);
-  p.tok_per_wg = append_tok_per_wg(n_tok, (int32_t)rows);
   p.err = ctx->err_word;
   p.claim = pool->claim;
   p.epoch = pool->claim ? pool->next_epoch() : 0u;
-  const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
   if ((rc = set_device(ctx))) return rc;
-  return launch(ctx, name.c_str(), dim3((unsigned)((n_tok + p.tok_per_wg - 1) / p.tok_per_wg), rows), dim3(128), p,
-                stream);
+  return launch_append(ctx, pool, p, stream);
 }
 
 // Size the context's own split-K workspace grows to when it holds `cur` bytes
@@ -1041,10 +1063,7 @@ namespace {
 // slots derived in the kernel (the unfused half of vk_append_decode).
 // Whether the decode launch of this plan appends the new tokens itself
 // (vk_append_decode): I8_BLK pools under the workgroup split or stream-K, fp16
-// pools for ragged batches under either, and any pool for one sequence under the
-// workgroup split, over tiles the folded kernels are built for. Several sequences
-// of the other types keep the append launch: the call may list one sequence at
-// two lengths, and the longer row must see the shorter one's token.
+// pools under stream-K, over tiles the folded kernels are built for.
 bool plan_folds_append(const vk_pool* pool, const vk_decode_args* a, const DecodePlan& pl) {
   const int kvt = pool->desc.kv_type;
   const bool alone = a->n_seqs == 1 && pl.wg_waves > 0;
@@ -1087,11 +1106,9 @@ int append_new_tokens(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, const
   p.bt_rows = pl.bt_rows;
   p.cap_tokens = a->max_context_len;
   p.n_tok = a->n_seqs;
-  p.tok_per_wg = append_tok_per_wg(a->n_seqs, pool->desc.n_kv_heads);
   p.err = ctx->err_word;
   p.claim = pool->claim;
   p.epoch = pool->claim ? pool->next_epoch() : 0u;
-  unsigned rows = (unsigned)pool->desc.n_kv_heads;
   if (rope.style != ROPE_NONE) {  // positions derived (context_len - 1); q rotated into q_out
     p.rope = rope.style;
     p.positions = nullptr;
@@ -1101,11 +1118,8 @@ int append_new_tokens(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, const
     p.q = const_cast<void*>(a->q);
     p.q_out = q_out;
     p.q_dtype = a->q_dtype;
-    rows += (unsigned)((a->n_heads + 1) / 2);
   }
-  const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
-  return launch(ctx, name.c_str(), dim3((unsigned)((a->n_seqs + p.tok_per_wg - 1) / p.tok_per_wg), rows), dim3(128),
-                p, stream);
+  return launch_append(ctx, pool, p, stream);
 }
 
 // vk_paged_decode, and with k_new the append of vk_append_decode as a launch
@@ -1119,9 +1133,10 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
   if (a->n_seqs == 0) return VK_OK;
   if (!a->q || !a->out || !a->context_lens) return fail(VK_ERR_BAD_ARG, "null device pointer");
   if ((rc = set_device(ctx))) return rc;
-  // plan_folds_append: the append inside the decode launch (the wave that holds a
-  // sequence's last block appends the token before loading it); every other plan
-  // appends in a launch of its own first
+  // I8_BLK pools under the workgroup split or stream-K, and fp16 pools under
+  // stream-K, take the append inside the decode launch (the wave that holds a
+  // sequence's last block appends the token before loading it); every other
+  // plan appends in a launch of its own first
   const int kvt = pool->desc.kv_type;
   const bool fold = k_new && plan_folds_append(pool, a, pl);
   const bool rope_fold = fold && rope.style != ROPE_NONE && plan_folds_rope(pool, a, pl);

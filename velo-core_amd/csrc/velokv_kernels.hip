@@ -972,8 +972,6 @@ DEV uint32_t tile_elem(int tok, int d, int esz, int D) {
   return (uint32_t)(tok * D + d) * esz;
 }
 
-DEV int clamp127(float r) { return (int)fminf(fmaxf(r, -127.f), 127.f); }
-
 // The I8_BLK rule for one new token x (dims 2*lane, 2*lane + 1) at offset o of
 // a block whose scale is s_old:
 //   s_new = max(s_old, fp16(amax / 127))
@@ -989,24 +987,41 @@ DEV float blk_scale(float s_old, uint16_t& s_bits, float x0, float x1) {
   }
   return s_old;
 }
-DEV int blk_requant(int c, float s_old, float s_new) { return clamp127(__builtin_rintf(((float)c * s_old) / s_new)); }
-DEV int blk_code(float x, float s_new) { return (s_new > 0.f) ? clamp127(__builtin_rintf(x / s_new)) : 0; }
+// The rule divides many values by one scale. x / s is taken as q = x y corrected
+// once by its exact remainder, y = 1 / s divided out once per scale: with y
+// correctly rounded and q within an ulp that is the correctly rounded quotient
+// (Markstein, IBM J. Res. Dev. 34, 1990), in three instructions where the full
+// division takes about ten; checked against x / s for every fp16 scale, values
+// around every rounding tie among them. A scale past fp16's range is infinite
+// (values past 8.3e6) and takes the division: its remainder would be 0 x inf.
+DEV float blk_inv(float s) { return 1.0f / s; }
+DEV float div_scale(float x, float s, float y) {
+  const float q = x * y;
+  return fmaf(fmaf(-q, s, x), y, q);
+}
+DEV float blk_rne(float x, float s, float y) {
+  const float q = s < __builtin_huge_valf() ? div_scale(x, s, y) : x / s;  // (wave-uniform)
+  return fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f);
+}
+DEV int blk_requant(int c, float s_old, float s_new, float y) { return (int)blk_rne((float)c * s_old, s_new, y); }
+DEV int blk_code(float x, float s_new, float y) { return s_new > 0.f ? (int)blk_rne(x, s_new, y) : 0; }
 
 // The rule over a block whose codes are in registers (cd) and whose scale is
 // s_old (bits s_bits).
 DEV void blk_put(int (&cd)[BS][2], int o, float& s_old, uint16_t& s_bits, float x0, float x1) {
   const float s_new = blk_scale(s_old, s_bits, x0, x1);
+  const float y = blk_inv(s_new);
   if (s_new > s_old && o > 0) {
 #pragma unroll
     for (int u = 0; u < BS; ++u) {
       if (u < o) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k) cd[u][k] = blk_requant(cd[u][k], s_old, s_new);
+        for (int k = 0; k < 2; ++k) cd[u][k] = blk_requant(cd[u][k], s_old, s_new, y);
       }
     }
   }
-  const int c0 = blk_code(x0, s_new);
-  const int c1 = blk_code(x1, s_new);
+  const int c0 = blk_code(x0, s_new, y);
+  const int c1 = blk_code(x1, s_new, y);
 #pragma unroll
   for (int u = 0; u < BS; ++u)
     if (u == o) { cd[u][0] = c0; cd[u][1] = c1; }
@@ -1101,15 +1116,15 @@ DEV int byte_at(uint32_t w, int k) { return (int)(int8_t)(uint8_t)(w >> (8 * k))
 // 64-dim row read the codes 64 dims below and store nothing. K codes of token u
 // at dims 2 lane, 2 lane + 1 are two adjacent bytes; V codes of the token pair
 // 2p, 2p + 1 are four (dim 2 lane: tokens 2p, 2p + 1; then dim 2 lane + 1).
-DEV uint32_t blk_requant4(uint32_t w, float s_old, float s_new) {
+DEV uint32_t blk_requant4(uint32_t w, float s_old, float s_new, float y) {
   uint32_t r = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) r |= (uint32_t)(blk_requant(byte_at(w, k), s_old, s_new) & 0xFF) << (8 * k);
+  for (int k = 0; k < 4; ++k) r |= (uint32_t)(blk_requant(byte_at(w, k), s_old, s_new, y) & 0xFF) << (8 * k);
   return r;
 }
-DEV uint4 blk_requant16(uint4 v, float s_old, float s_new) {
-  return make_uint4(blk_requant4(v.x, s_old, s_new), blk_requant4(v.y, s_old, s_new), blk_requant4(v.z, s_old, s_new),
-                    blk_requant4(v.w, s_old, s_new));
+DEV uint4 blk_requant16(uint4 v, float s_old, float s_new, float y) {
+  return make_uint4(blk_requant4(v.x, s_old, s_new, y), blk_requant4(v.y, s_old, s_new, y),
+                    blk_requant4(v.z, s_old, s_new, y), blk_requant4(v.w, s_old, s_new, y));
 }
 
 template <bool IS_V, int D>
@@ -1125,14 +1140,15 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
   const float s_new = blk_scale(s_old, s_bits, f.x[e][0], f.x[e][1]);
   const bool grew = s_new > s_old && o > 0;  // requantize the tokens before o
   uint8_t* tile = const_cast<uint8_t*>(IS_V ? P.vc : P.kc) + f.tix * P.tile_bytes;
-  const int c0 = blk_code(f.x[e][0], s_new), c1 = blk_code(f.x[e][1], s_new);
+  const float y = blk_inv(s_new);
+  const int c0 = blk_code(f.x[e][0], s_new, y), c1 = blk_code(f.x[e][1], s_new, y);
   if constexpr (!IS_V) {
     if (grew) {
 #pragma unroll
       for (int j = 0; j < D / 64; ++j) {
         const int q = lane + 64 * j;
         if ((q % (D / 2)) / (D / 32) < o)  // the piece's token
-          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.kq[j], s_old, s_new);
+          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.kq[j], s_old, s_new, y);
       }
     }
     if (st)
@@ -1143,7 +1159,7 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
       for (int j = 0; j < D / 64; ++j) {
         const int q = lane + 64 * j;
         if (q / (D / 8) < (o >> 1))  // the piece's token pair
-          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.vq[j], s_old, s_new);
+          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.vq[j], s_old, s_new, y);
       }
     }
     if (st) {  // bytes: (2P, d0), (2P + 1, d0), (2P, d0 + 1), (2P + 1, d0 + 1)
@@ -1151,8 +1167,8 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
       if (o & 1) {  // token o - 1 (requantized when the scale grew), then token o
         int a0 = byte_at(w, 0), a1 = byte_at(w, 2);
         if (grew) {
-          a0 = blk_requant(a0, s_old, s_new);
-          a1 = blk_requant(a1, s_old, s_new);
+          a0 = blk_requant(a0, s_old, s_new, y);
+          a1 = blk_requant(a1, s_old, s_new, y);
         }
         w = (uint32_t)(a0 & 0xFF) | ((uint32_t)(c0 & 0xFF) << 8) | ((uint32_t)(a1 & 0xFF) << 16) |
             ((uint32_t)(c1 & 0xFF) << 24);
@@ -2916,24 +2932,47 @@ DEV int rope_pos(const AppendParams& P, int m) {
 
 // Flat slot of token m, or -1 when it is padding (a negative slot, or one at or
 // past the end of the pool) or, with RoPE, its position is outside the table.
-DEV int64_t token_slot(const AppendParams& P, int m) {
+// token_in loads what the call holds of it (its slot and position, or its
+// sequence's length; a word that exists in the place of the others), in no branch,
+// so that they go out with a caller's other loads: the compiler waits for the loads
+// in a branch at its end. token_slot_of puts them together with the table entry.
+struct TokenIn {
   int64_t slot;
-  if (P.slot_mapping) {
-    slot = P.slot_mapping[m];
-  } else {  // the new token of sequence m, at its last context position (kernels.metal:770-774)
-    const int pos = min(P.context_lens[m], P.cap_tokens) - 1;
+  int pos, ctx;
+};
+DEV TokenIn token_in(const AppendParams& P, int m) {
+  TokenIn t;
+  t.slot = P.slot_any[P.slot_mapping ? m : 0];
+  t.pos = P.pos_any[P.positions ? m : 0];
+  t.ctx = P.ctx_any[P.slot_mapping ? 0 : m];
+  return t;
+}
+DEV int new_pos(const AppendParams& P, const TokenIn& t) { return min(t.ctx, P.cap_tokens) - 1; }
+DEV int pos_of(const AppendParams& P, const TokenIn& t) { return P.positions ? t.pos : new_pos(P, t); }
+// Table entry of the new token of sequence m, at its last context position
+// (kernels.metal:770-774); -1 when the row has no such entry.
+DEV int token_entry(const AppendParams& P, int m, const TokenIn& t) {
+  if (P.slot_mapping) return -1;
+  const int pg = new_pos(P, t) / (BS * P.g.page_tiles);
+  if (new_pos(P, t) < 0 || pg >= P.bt_stride) return -1;
+  int row = m;
+  if (P.seq_rows) row = P.seq_rows[m];
+  if (P.bt_rows > 0) row = min(max(row, 0), P.bt_rows - 1);
+  return P.block_tables[(int64_t)row * P.bt_stride + pg];
+}
+DEV int64_t token_slot_of(const AppendParams& P, const TokenIn& t, int entry) {
+  int64_t slot = t.slot;
+  if (!P.slot_mapping) {
     const int ptok = BS * P.g.page_tiles;  // the page's tokens
-    if (pos < 0 || pos / ptok >= P.bt_stride) return -1;
-    int row = P.seq_rows ? P.seq_rows[m] : m;
-    if (P.bt_rows > 0) row = min(max(row, 0), P.bt_rows - 1);
-    slot = (int64_t)P.block_tables[(int64_t)row * P.bt_stride + pos / ptok] * ptok + pos % ptok;
+    slot = entry < 0 ? -1 : (int64_t)entry * ptok + new_pos(P, t) % ptok;
   }
   if (slot < 0 || slot >= (int64_t)P.g.n_blocks * BS) return -1;
-  if (P.rope != ROPE_NONE) {
-    const int pos = rope_pos(P, m);
-    if (pos < 0 || pos >= P.n_pos) return -1;
-  }
+  if (P.rope != ROPE_NONE && (pos_of(P, t) < 0 || pos_of(P, t) >= P.n_pos)) return -1;
   return slot;
+}
+DEV int64_t token_slot(const AppendParams& P, int m) {
+  const TokenIn t = token_in(P, m);
+  return token_slot_of(P, t, token_entry(P, m, t));
 }
 
 // K/V row elements (dims 2l, 2l+1) of token m, head h, rotated for K when RoPE is on.
@@ -2972,6 +3011,7 @@ DEV int prev_block(const AppendParams& P, int n) {
 // The run that starts at token w0 + j (slot `slot`), for KV head h; ms0 holds
 // the slots of tokens w0 .. w0 + 63 (lane i: token w0 + i, -1 past the end), so
 // the first step of the run's forward scan needs no load.
+constexpr int kRunBatch = 4;
 template <bool IS_V, int D>
 DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int w0, int j,
                         int64_t slot, int64_t ms0, int h) {
@@ -3011,9 +3051,10 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
       cd[u][1] = (int8_t)(uint8_t)(w >> 8);
     }
   }
-  const uint16_t stored = *sp;
-  float s_old = 0.f;
-  uint16_t s_bits = 0;
+  // the running scale as fp16 bits in a scalar: scales are never negative, so
+  // their bits order as they do
+  const int stored = __builtin_amdgcn_readfirstlane((int)*sp);
+  int s_bits = 0;
   int hi_written = -1;
   bool first = true;
   for (int base = w0; base < P.n_tok; base += WAVE) {
@@ -3031,7 +3072,7 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
       // once the running scales are known the new codes) is computed for all
       // members at once; only the running scale and the placement, with its
       // requantization when the scale grew, follow the members' order.
-      constexpr int kBatch = 8;
+      constexpr int kBatch = kRunBatch;
       float xs[kBatch][2];
       int ok[kBatch];  // member offsets in the block (wave-uniform)
       int nb = 0;
@@ -3050,54 +3091,48 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
         }
         mem = rest;
       }
-      uint16_t cand[kBatch];  // fp16(amax / 127) of each member (wave-uniform)
+      // the scale before (so) and after (sn) each member: fp16 bits, from the
+      // member's fp16(amax / 127) (amax counts no NaN)
+      int so[kBatch], sn[kBatch];
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
-        cand[k] = 0;
+        sn[k] = 0;
         if (k < nb) {
-          const float amax = wave_max(fmaxf(fabsf(xs[k][0]), fabsf(xs[k][1])));
-          cand[k] = (uint16_t)__builtin_amdgcn_readfirstlane((int)f2h(amax / 127.0f));
+          const float amax = wave_max(fmaxf(fmaxf(0.f, fabsf(xs[k][0])), fabsf(xs[k][1])));
+          sn[k] = __builtin_amdgcn_readfirstlane((int)f2h(amax / 127.0f));
         }
       }
-      // the scale before (so) and after (sn) each member
-      float so[kBatch], sn[kBatch];
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
-        so[k] = sn[k] = 0.f;
+        so[k] = 0;
         if (k < nb) {
           const int o = ok[k];
-          if (first) {
-            s_old = (o == 0) ? 0.f : h2f(stored);
-            s_bits = (o == 0) ? (uint16_t)0 : stored;
-            first = false;
-          } else if (o == 0) {
-            s_old = 0.f;
-            s_bits = 0;
-          }
-          so[k] = s_old;
-          if (h2f(cand[k]) > s_old) {
-            s_bits = cand[k];
-            s_old = h2f(cand[k]);
-          }
-          sn[k] = s_old;
+          if (o == 0) s_bits = 0;
+          else if (first) s_bits = stored;
+          first = false;
+          so[k] = s_bits;
+          s_bits = max(s_bits, sn[k]);
+          sn[k] = s_bits;
         }
       }
       int cc[kBatch][2];
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
-        cc[k][0] = k < nb ? blk_code(xs[k][0], sn[k]) : 0;
-        cc[k][1] = k < nb ? blk_code(xs[k][1], sn[k]) : 0;
+        const float s_k = h2f((uint16_t)sn[k]), y = blk_inv(s_k);
+        cc[k][0] = k < nb ? blk_code(xs[k][0], s_k, y) : 0;
+        cc[k][1] = k < nb ? blk_code(xs[k][1], s_k, y) : 0;
       }
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
         if (k < nb) {
           const int o = ok[k];
           if (sn[k] > so[k] && o > 0) {
+            const float s_o = h2f((uint16_t)so[k]), s_k = h2f((uint16_t)sn[k]), y = blk_inv(s_k);
 #pragma unroll
             for (int u = 0; u < BS; ++u) {
               if (u < o) {
-                cd[u][0] = blk_requant(cd[u][0], so[k], sn[k]);
-                cd[u][1] = blk_requant(cd[u][1], so[k], sn[k]);
+                cd[u][0] = blk_requant(cd[u][0], s_o, s_k, y);
+                cd[u][1] = blk_requant(cd[u][1], s_o, s_k, y);
               }
             }
           }
@@ -3125,16 +3160,208 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
       if (din && u <= hi_written)
         *reinterpret_cast<uint16_t*>(lp0 + tile_elem<false>(u, 0, 1, D)) = (uint16_t)(b8(cd[u][0]) | (b8(cd[u][1]) << 8));
   }
-  if (lane == 0) *sp = s_bits;
+  if (lane == 0) *sp = (uint16_t)s_bits;
+}
+
+// Caller rows (K, V, q) are read in 16-byte pieces whatever their alignment above
+// the element's: the hardware takes any 4-byte address.
+typedef uint32_t u32x4_in __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_in __attribute__((ext_vector_type(2), aligned(4)));
+// ND dims d0 .. of NT caller rows (element offsets) as fp32, dims past io read as
+// the first ones; the loads of all in one branch on the type (the compiler waits
+// for a branch's loads at its end).
+template <int NT, int ND>
+DEV void load_x8n(const void* src, int in_dtype, const int64_t (&row)[NT], int d0, int io, float (&x)[NT][ND]) {
+  if (in_dtype == DT_F16) {
+    const uint16_t* s = reinterpret_cast<const uint16_t*>(src);
+    u32x4 w[NT][ND / 8];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < ND / 8; ++e)
+        w[i][e] = *reinterpret_cast<const u32x4_in*>(s + row[i] + (d0 + 8 * e < io ? d0 + 8 * e : 0));
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int k = 0; k < ND / 2; ++k) {
+        x[i][2 * k] = half_lo(w[i][k >> 2][k & 3]);
+        x[i][2 * k + 1] = half_hi(w[i][k >> 2][k & 3]);
+      }
+  } else {
+    const float* s = reinterpret_cast<const float*>(src);
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < ND / 4; ++e) {
+        const u32x4 w = *reinterpret_cast<const u32x4_in*>(s + row[i] + (d0 + 4 * e < io ? d0 + 4 * e : 0));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[i][4 * e + k] = __uint_as_float(w[k]);
+      }
+  }
+}
+// RoPE of a lane's ND dims d0 .. of a token's K row at position pos (rope_rotate's
+// expressions and order). Half-split partners, io_hd / 2 dims away, are in the
+// lane two away of the token's four (called only with io_hd the tile width D).
+template <int ND, int D>
+DEV void rope_tile_rows(const AppendParams& P, int pos, int d0, float (&x)[ND]) {
+#pragma clang fp contract(off)
+  const int io = P.g.io_hd;
+  const float* cs = P.cos_sin + (int64_t)pos * io;
+  if (P.rope == ROPE_INTERLEAVED) {
+#pragma unroll
+    for (int k = 0; k < ND; k += 4) {
+      const float4 t = *reinterpret_cast<const float4*>(cs + (d0 + k < io ? d0 + k : 0));
+      if (d0 + k < io) {
+        const float a = x[k], b = x[k + 1], c = x[k + 2], d = x[k + 3];
+        x[k] = a * t.x - b * t.y;
+        x[k + 1] = a * t.y + b * t.x;
+        x[k + 2] = c * t.z - d * t.w;
+        x[k + 3] = c * t.w + d * t.z;
+      }
+    }
+  } else {
+    const bool first = d0 < D / 2;
+    cs += 2 * (first ? d0 : d0 - D / 2);
+#pragma unroll
+    for (int k = 0; k < ND; k += 2) {
+      const float4 t = *reinterpret_cast<const float4*>(cs + 2 * k);
+      const float p0 = dpp<DPP_QUAD_XOR2>(x[k]), p1 = dpp<DPP_QUAD_XOR2>(x[k + 1]);
+      x[k] = first ? x[k] * t.x - p0 * t.y : p0 * t.y + x[k] * t.x;
+      x[k + 1] = first ? x[k + 1] * t.z - p1 * t.w : p1 * t.w + x[k + 1] * t.z;
+    }
+  }
+}
+
+DEV uint32_t pack_i8x4(float a, float b, float c, float d) {
+  return ((uint32_t)(int)a & 0xFFu) | (((uint32_t)(int)b & 0xFFu) << 8) | (((uint32_t)(int)c & 0xFFu) << 16) |
+         ((uint32_t)(int)d << 24);
+}
+
+// A run of m tokens n0 .. n0 + m - 1 of the call in the consecutive slots o0 ..
+// of block b (a prompt's blocks, a draft's tokens, one new token): the rule of
+// append_blk_run with every step over all tokens of the block at once. K lane 4 t + c
+// holds the D / 4 dims of token t that its 16-byte pieces of the tile hold, V lane
+// 8 p + c D / 8 dims of the token pair p. The running scales are a prefix maximum
+// of the tokens' fp16 candidates (scales are never negative, so their bits order
+// as they do), the stored scale standing for the tokens before o0; each token
+// where it grows re-codes the lanes of the tokens before. The rows and, unless
+// the run fills the block, the block's codes and scale are one round trip.
+// Bound by that and by the vector ALUs (2.4 growths in a fresh block, 45
+// instructions each and lane), where a wave with two dims of every token went
+// through the tokens one after another: 8,000 tokens x 8 heads with 32 rotated
+// query heads 163 -> 53 us (K and V alone 53 -> 29), 2,048 draft tokens 23 -> 22.
+template <bool IS_V, int D>
+DEV void append_blk_tile(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int n0, int m, int o0,
+                         int64_t b, int h) {
+  constexpr int NV = D / 4;             // values per lane
+  constexpr int NT = IS_V ? 2 : 1;      // tokens per lane
+  constexpr int ND = NV / NT;           // dims per lane
+  constexpr int LT = WAVE / BS * NT;    // lanes that share a token (or a pair)
+  const int lane = lane_id();
+  const int t0 = lane / LT * NT, d0 = lane % LT * ND;
+  const int io = P.g.io_hd, Hkv = P.g.n_kv_heads;
+  uint8_t* tile = codes + ((uint64_t)b * Hkv + h) * P.g.tile_bytes;
+  uint16_t* sp = scales + ((uint64_t)b * Hkv + h) * (kBlkScaleStep / 2);
+  // (a run that fills the block reads nothing of it: descriptors of no bytes)
+  const rsrc_t tr = make_rsrc(tile, m < BS ? P.g.tile_bytes : 0u);
+  u32x4 old[NV / 16];  // the lane's 16-byte pieces
+#pragma unroll
+  for (int q = 0; q < NV / 16; ++q)
+    old[q] = __builtin_amdgcn_raw_buffer_load_b128(tr, (int)tile_elem<IS_V>(t0, d0 + q * 16 / NT, 1, D), 0, 0);
+  const int stored = o0 > 0 ? __builtin_amdgcn_readfirstlane((int)*sp) : 0;
+  float x[NT][ND];
+  bool mine[NT];  // token t0 + i is in the run
+  int64_t row[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int k = t0 + i - o0;
+    mine[i] = k >= 0 && k < m;
+    row[i] = ((int64_t)(n0 + (mine[i] ? k : 0)) * Hkv + h) * io;
+  }
+  load_x8n<NT, ND>(src, P.in_dtype, row, d0, io, x);
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int k = 0; k < ND; ++k) x[i][k] = mine[i] && d0 + (k & ~7) < io ? x[i][k] : 0.f;
+  if constexpr (!IS_V) {
+    const int n = n0 + (mine[0] ? t0 - o0 : 0);
+    if (P.rope != ROPE_NONE) {
+      rope_tile_rows<ND, D>(P, rope_pos(P, n), d0, x[0]);
+#pragma unroll
+      for (int k = 0; k < ND; ++k) x[0][k] = mine[0] ? x[0][k] : 0.f;
+    }
+  }
+  int bits[NT];  // candidate scale, then the scale after the token (fp16 bits)
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    float a = 0.f;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) a = fmaxf(a, fabsf(x[i][k]));
+    a = fmaxf(a, dpp<DPP_QUAD_XOR1>(a));
+    a = fmaxf(a, dpp<DPP_QUAD_XOR2>(a));
+    if constexpr (LT == 8) a = fmaxf(a, dpp<DPP_ROW_HALF_MIRROR>(a));
+    bits[i] = max(stored, (int)f2h(a / 127.0f));
+  }
+  int pre = NT == 2 ? max(bits[0], bits[NT - 1]) : bits[0];
+  if constexpr (LT == 4) pre = max(pre, __builtin_amdgcn_update_dpp(0, pre, 0x114, 0xF, 0xF, false));  // row_shr 4
+  pre = max(pre, __builtin_amdgcn_update_dpp(0, pre, 0x118, 0xF, 0xF, false));                         // row_shr 8
+  pre = max(pre, __builtin_amdgcn_update_dpp(0, pre, 0x142, 0xA, 0xF, false));                         // row_bcast 15
+  pre = max(pre, __builtin_amdgcn_update_dpp(0, pre, 0x143, 0xC, 0xF, false));                         // row_bcast 31
+  if constexpr (NT == 2) {
+    const int before = __shfl_up(pre, LT, WAVE);
+    bits[0] = max(lane < LT ? 0 : before, bits[0]);
+  }
+  bits[NT - 1] = pre;
+  float c[NT][ND];  // codes: the run's tokens', and as stored the others'
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const float s = h2f((uint16_t)bits[i]), y = blk_inv(s);
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      const int byte = IS_V ? 2 * k + i : k;
+      const float was = byte_to_f(old[byte / 16][byte / 4 % 4], byte % 4);
+      const float now = s > 0.f ? blk_rne(x[i][k], s, y) : 0.f;
+      c[i][k] = mine[i] ? now : was;
+    }
+  }
+  int s_prev = stored;
+#pragma unroll 1
+  for (int u = o0; u < o0 + m; ++u) {
+    const int l = u / NT * LT;
+    const int s_u = NT == 2 && (u & 1) ? readlane_i(bits[NT - 1], l) : readlane_i(bits[0], l);
+    if (s_u > s_prev && u > 0) {  // token u grew the scale: the tokens before it take the new one
+      const float so = h2f((uint16_t)s_prev), sn = h2f((uint16_t)s_u), y = blk_inv(sn);
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+        if (t0 + i < u) {
+#pragma unroll
+          for (int k = 0; k < ND; ++k) c[i][k] = blk_rne(c[i][k] * so, sn, y);
+        }
+    }
+    s_prev = s_u;
+  }
+  uint32_t w[NV / 4];
+#pragma unroll
+  for (int k = 0; k < NV / 4; ++k)
+    w[k] = IS_V ? pack_i8x4(c[0][(2 * k) % ND], c[NT - 1][(2 * k) % ND], c[0][(2 * k + 1) % ND], c[NT - 1][(2 * k + 1) % ND])
+                : pack_i8x4(c[0][(4 * k) % ND], c[0][(4 * k + 1) % ND], c[0][(4 * k + 2) % ND], c[0][(4 * k + 3) % ND]);
+  // the pieces with a token of the run, and when the scale grew past the stored
+  // one those of the tokens before (a V pair's token past the run as it was)
+  if (t0 < o0 + m && (t0 + NT > o0 || s_prev > stored)) {
+#pragma unroll
+    for (int q = 0; q < NV / 16; ++q)
+      *reinterpret_cast<uint4*>(tile + tile_elem<IS_V>(t0, d0 + q * 16 / NT, 1, D)) =
+          make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
+  }
+  if (lane == 0) *sp = (uint16_t)s_prev;
 }
 
 // The runs that start inside tokens [w0, w0 + T) of the call, in order. A token
 // starts a run when it is not padding and the nearest non-padding token before
 // it is in another block (or there is none).
 template <bool IS_V, int D>
-DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int w0, int T) {
+DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int w0, int T, int h) {
   const int lane = lane_id();
-  const int h = blockIdx.y;
   const int m = w0 + lane;
   // slots of 64 tokens from w0: the window's T and what follows (reused by the runs' forward scans)
   const int64_t ms64 = m < P.n_tok ? token_slot(P, m) : -1;
@@ -3162,120 +3389,317 @@ DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint
     const unsigned long long me = ((unsigned long long)P.epoch << 32) | (uint32_t)(w0 + j);
     unsigned long long old = 0;
     if (claim) old = __hip_atomic_exchange(&P.claim[slot / BS], me, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    append_blk_run<IS_V, D>(P, src, codes, scales, w0, j, slot, ms64, h);
+    // tokens in consecutive slots of the block, and nothing of the block after them
+    // (the block's end, the call's end or a token of another block; no padding or
+    // reordering within): all at once (a half-split rotation needs its partners in
+    // the lanes that path gives them; one token is done sooner with its dims over
+    // the wave, 5.4 us a call against 7.4)
+    const int o0 = (int)(slot % BS);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(lane >= j && ms64 == slot + (lane - j)) >> j;
+    const int m = min(BS - o0, __builtin_ctzll(~same));
+    const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m < 64
+    const int nx = __shfl((int)(ms64 / BS), after != 0 ? j + m + __builtin_ctzll(after) : 0, WAVE);
+    if (m > 1 && (o0 + m == BS || (after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok)) &&
+        (IS_V || P.rope != ROPE_HALF || P.g.io_hd == D))
+      append_blk_tile<IS_V, D>(P, src, codes, scales, w0 + j, m, o0, slot / BS, h);
+    else
+      append_blk_run<IS_V, D>(P, src, codes, scales, w0, j, slot, ms64, h);
     if (claim && (uint32_t)(old >> 32) == P.epoch && old != me) flag_misuse(P.err, MISUSE_BLK_SPLIT_RUN);
   }
 }
 
-// VK_KV_I8_REF: per-(token, head) fp32 scale = amax/127, codes = trunc(x * (127/amax)).
-template <bool IS_V>
-DEV void append_ref(const AppendParams& P, const void* src, uint8_t* codes, float* scales, int n, int64_t slot) {
-  const int lane = lane_id();
-  const int h = blockIdx.y;
-  if (slot < 0) return;
-  const int64_t b = slot / BS;
-  const int o = (int)(slot % BS);
-  if (b >= P.g.n_blocks) return;
-  const int Hkv = P.g.n_kv_heads;
-  const int d0 = 2 * lane;
-  float x0, x1;
-  load_kv(P, src, IS_V, n, h, x0, x1);
-  const float amax = wave_max(fmaxf(fabsf(x0), fabsf(x1)));
-  const float scale = amax / 127.0f;
-  const float inv = amax > 0.f ? 127.0f / amax : 0.f;
-  uint8_t* tile = codes + ((uint64_t)b * Hkv + h) * P.g.tile_bytes;
-  const int D = P.g.head_dim;
-  if (d0 < D) {
-    tile[tile_elem<IS_V>(o, d0, 1, D)] = (uint8_t)(int8_t)(int)(x0 * inv);
-    tile[tile_elem<IS_V>(o, d0 + 1, 1, D)] = (uint8_t)(int8_t)(int)(x1 * inv);
-  }
-  if (lane == 0) scales[((uint64_t)b * Hkv + h) * BS + o] = scale;
-}
+// ---- rows that are stored by themselves: q, and K and V of every type but I8_BLK
+// Sixteen lanes take a row: lane i < io_hd / 8 its dims 4 i .. 4 i + 3 and those
+// io_hd / 2 further on (so that the half-split rotation's partners are the
+// lane's own), the next lanes eight of the zero dims that pad it to the tile
+// width. A wave takes four tokens and row_batch query heads, with the loads of all
+// of them in flight and one read of the token's table row; a workgroup of two
+// waves eight tokens. Bound by memory from a few thousand tokens on; one token of
+// one head per wave and turn, as this was, waits out a memory round trip per row:
+// fp16, 8 K/V and 32 query heads, 777 tokens 12.6 -> 6.0 us, 8,000 tokens 115 -> 48.
+// VK_KV_I8_REF: per-(token, head) fp32 scale amax / 127, codes trunc(x * (127 / amax)).
+// V tiles interleave token pairs: where the call's next token is the second of
+// this one's pair (a prompt's tokens) this lane group writes both, in whole words.
+struct Row8 { float x[8]; };  // dims a .. a + 3, b .. b + 3
 
-// VK_KV_F16 / VK_KV_F32: plain copy (with RNE conversion to fp16 when needed).
-template <bool IS_V, int ESZ>
-DEV void append_plain(const AppendParams& P, const void* src, uint8_t* codes, int n, int64_t slot) {
-  const int lane = lane_id();
-  const int h = blockIdx.y;
-  if (slot < 0) return;
-  const int64_t b = slot / BS;
-  const int o = (int)(slot % BS);
-  if (b >= P.g.n_blocks) return;
-  const int Hkv = P.g.n_kv_heads;
-  const int d0 = 2 * lane;
-  uint8_t* tile = codes + ((uint64_t)b * Hkv + h) * P.g.tile_bytes;
-  const int D = P.g.head_dim;
-  if (ESZ == 2 && P.in_dtype == DT_F16 && (IS_V || P.rope == ROPE_NONE) && D == HD && P.g.io_hd == HD) {
-    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(src) + ((int64_t)n * Hkv + h) * HD + d0;
-    *reinterpret_cast<uint16_t*>(tile + tile_elem<IS_V>(o, d0, 2, HD)) = s16[0];
-    *reinterpret_cast<uint16_t*>(tile + tile_elem<IS_V>(o, d0 + 1, 2, HD)) = s16[1];
-    return;
-  }
-  float x0, x1;
-  load_kv(P, src, IS_V, n, h, x0, x1);
-  if (d0 >= D) return;
-  if constexpr (ESZ == 2) {
-    *reinterpret_cast<uint16_t*>(tile + tile_elem<IS_V>(o, d0, 2, D)) = f2h(x0);
-    *reinterpret_cast<uint16_t*>(tile + tile_elem<IS_V>(o, d0 + 1, 2, D)) = f2h(x1);
+// N rows of io elements (element offsets `row`) of src at the lane's dims. All
+// loads of the rows go out in one branch on the type: the compiler waits for a
+// branch's loads at its end, so a branch per row was a round trip per row.
+template <int N>
+DEV void load_rows8(const void* src, int dtype, const int64_t (&row)[N], int a, int b, bool in, Row8 (&r)[N]) {
+  const int oa = in ? a : 0, ob = in ? b : 0;
+  if (dtype == DT_F16) {
+    const auto s = (const __attribute__((address_space(1))) uint16_t*)src;
+    u32x2 w[N][2];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      w[j][0] = *(const __attribute__((address_space(1))) u32x2_in*)(s + row[j] + oa);
+      w[j][1] = *(const __attribute__((address_space(1))) u32x2_in*)(s + row[j] + ob);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        r[j].x[2 * k] = half_lo(w[j][k >> 1][k & 1]);
+        r[j].x[2 * k + 1] = half_hi(w[j][k >> 1][k & 1]);
+      }
   } else {
-    *reinterpret_cast<float*>(tile + tile_elem<IS_V>(o, d0, 4, D)) = x0;
-    *reinterpret_cast<float*>(tile + tile_elem<IS_V>(o, d0 + 1, 4, D)) = x1;
+    const auto s = (const __attribute__((address_space(1))) float*)src;
+    u32x4 w[N][2];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      w[j][0] = *(const __attribute__((address_space(1))) u32x4_in*)(s + row[j] + oa);
+      w[j][1] = *(const __attribute__((address_space(1))) u32x4_in*)(s + row[j] + ob);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) r[j].x[k] = __uint_as_float(w[j][k >> 2][k & 3]);
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[j].x[k] = in ? r[j].x[k] : 0.f;
+}
+// rope_rotate of the lane's dims, t0 and t1 the table's pairs of dims a .. and b ..
+// (interleaved) or the first and last two pairs of a .. a + 3 (half-split).
+DEV void rope_row8(Row8& r, int style, const float4 t0, const float4 t1) {
+#pragma clang fp contract(off)
+  float* x = r.x;
+  if (style == ROPE_INTERLEAVED) {
+    const float a0 = x[0], a1 = x[1], a2 = x[2], a3 = x[3], b0 = x[4], b1 = x[5], b2 = x[6], b3 = x[7];
+    x[0] = a0 * t0.x - a1 * t0.y; x[1] = a0 * t0.y + a1 * t0.x;
+    x[2] = a2 * t0.z - a3 * t0.w; x[3] = a2 * t0.w + a3 * t0.z;
+    x[4] = b0 * t1.x - b1 * t1.y; x[5] = b0 * t1.y + b1 * t1.x;
+    x[6] = b2 * t1.z - b3 * t1.w; x[7] = b2 * t1.w + b3 * t1.z;
+  } else {
+    const float c[4] = {t0.x, t0.z, t1.x, t1.z}, sn[4] = {t0.y, t0.w, t1.y, t1.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float u = x[k], v = x[4 + k];
+      x[k] = u * c[k] - v * sn[k];
+      x[4 + k] = u * sn[k] + v * c[k];
+    }
   }
 }
+DEV float max16(float m) {  // over the row's sixteen lanes
+  m = fmaxf(m, dpp<DPP_QUAD_XOR1>(m));
+  m = fmaxf(m, dpp<DPP_QUAD_XOR2>(m));
+  m = fmaxf(m, dpp<DPP_ROW_HALF_MIRROR>(m));
+  return fmaxf(m, dpp<DPP_ROW_MIRROR>(m));
+}
+// The stored form of a row: fp16 or fp32 values, or the I8_REF codes (and scale).
+template <int KV>
+DEV void row_codes(const Row8& r, uint32_t (&w)[8], float& scale) {
+  if constexpr (KV == KV_I8_REF) {
+    float m = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(r.x[k]));
+    m = max16(m);
+    scale = m / 127.0f;
+    const float inv = m > 0.f ? 127.0f / m : 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = (uint32_t)(uint8_t)(int8_t)(int)(r.x[k] * inv);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = KV == KV_F16 ? (uint32_t)f2h(r.x[k]) : __float_as_uint(r.x[k]);
+  }
+}
+template <int ESZ>
+DEV void store4(uint8_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  if constexpr (ESZ == 4) *reinterpret_cast<uint4*>(p) = make_uint4(a, b, c, d);
+  else if constexpr (ESZ == 2) *reinterpret_cast<uint2*>(p) = make_uint2(a | (b << 16), c | (d << 16));
+  else *reinterpret_cast<uint32_t*>(p) = a | (b << 8) | (c << 16) | (d << 24);
+}
+template <int ESZ>
+DEV void store1(uint8_t* p, uint32_t a) {
+  if constexpr (ESZ == 4) *reinterpret_cast<uint32_t*>(p) = a;
+  else if constexpr (ESZ == 2) *reinterpret_cast<uint16_t*>(p) = (uint16_t)a;
+  else *p = (uint8_t)a;
+}
 
-// D: head_dim of the pool for the I8_BLK rule (a compile-time constant, so that
-// the 16 tokens' tile offsets fold into the instructions; vk_append_kv3 / _d64).
-template <int KV, int D = HD>
-DEV void append_kernel(const AppendParams& P) {
-  const int T = P.tok_per_wg;
-  const int w0 = (int)blockIdx.x * T;
-  const int w1 = min(w0 + T, P.n_tok);
-  if ((int)blockIdx.y >= P.g.n_kv_heads) {  // RoPE of two query heads of the window's tokens
-    const int head = 2 * ((int)blockIdx.y - P.g.n_kv_heads) + (int)(threadIdx.x / WAVE);
-    if (head >= P.n_heads) return;
-    void* qd = P.q_out ? P.q_out : P.q;
-    for (int n = w0; n < w1; ++n) {
-      const int pos = rope_pos(P, n);
-      const int64_t off = ((int64_t)n * P.n_heads + head) * P.g.io_hd + 2 * lane_id();
-      float x0 = 0.f, x1 = 0.f;
-      const bool in = 2 * lane_id() < P.g.io_hd;
-      if (in) load_x2(P.q, P.q_dtype, off, x0, x1);
-      const bool rot = pos >= 0 && pos < P.n_pos;  // (wave-uniform)
-      if (rot) rope_rotate(P.rope, P.cos_sin, pos, P.g.io_hd, x0, x1);
-      if (!in || (!rot && !P.q_out)) continue;  // unrotated rows stay as they are (copied when q_out is given)
-      if (P.q_dtype == DT_F16) {
-        reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(qd) + off)[0] =
-            (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
-      } else {
-        reinterpret_cast<float2*>(reinterpret_cast<float*>(qd) + off)[0] = make_float2(x0, x1);
+// Row group grp (query heads, RB a group, then K heads, then V heads) of the
+// tokens 8 tg .. 8 tg + 7.
+template <int KV, int RB>
+DEV void append_rows(const AppendParams& P, int id) {
+  // The arguments that the first loads need, read together (one wait each for the
+  // lines they lie on otherwise), and the pointers as loaded values: a select between
+  // the loads became a select of their addresses, which kept a copy of the arguments
+  // in scratch memory.
+  const void *pq = P.q, *pk = P.k, *pv = P.v;
+  int tq = P.q_dtype, tk = P.in_dtype;
+  uint8_t* base = P.base;
+  __asm__ volatile("" : "+s"(pq), "+s"(pk), "+s"(pv), "+s"(tq), "+s"(tk), "+s"(base) : "s"(P.row_groups), "s"(P.g.n_kv_heads), "s"(P.slot_mapping), "s"(P.positions), "s"(P.slot_any), "s"(P.pos_any), "s"(P.ctx_any));
+  const int tg = (uint32_t)id / (uint32_t)P.row_groups, grp = id - tg * P.row_groups;
+
+  constexpr int ESZ = Esz<KV>::v;
+  const int lane = lane_id(), i = lane & 15;
+  const int n_raw = 8 * tg + 4 * (int)(threadIdx.x / WAVE) + (lane >> 4);
+  const bool tok = n_raw < P.n_tok;
+  const int n = min(n_raw, P.n_tok - 1);
+  const int io = P.g.io_hd, D = P.g.head_dim, Hkv = P.g.n_kv_heads;
+  const bool in = i < io / 8;
+  const int a = in ? 4 * i : io + 8 * (i - io / 8), b = in ? a + io / 2 : a + 4;
+  const int gq = (P.n_heads + RB - 1) / RB;
+  const bool is_q = KV == KV_I8_BLK || grp < gq, is_v = KV != KV_I8_BLK && grp >= gq + Hkv;
+  const int h = is_q ? RB * grp : is_v ? grp - gq - Hkv : grp - gq;
+  const int nh = is_q ? P.n_heads : Hkv;
+  const void* src = is_q ? pq : is_v ? pv : pk;
+  const int dtype = is_q ? tq : tk;
+  const int64_t row = (int64_t)n * nh + h;
+  if (is_v) {
+    if constexpr (KV != KV_I8_BLK) {
+      // both tokens of a pair by the first one's lanes when the call has them in a row
+      const bool more = n + 1 < P.n_tok;
+      const int n1 = more ? n + 1 : n, n0 = max(n - 1, 0);
+      const TokenIn t = token_in(P, n), t1 = token_in(P, n1), t0 = token_in(P, n0);
+      Row8 r[2];
+      const int64_t rows[2] = {row * io, (more ? row + nh : row) * io};
+      load_rows8<2>(src, dtype, rows, a, b, in, r);
+      // (new tokens of a batch's sequences, whose slots come from the table, go one by one)
+      const int64_t slot = tok ? token_slot_of(P, t, token_entry(P, n, t)) : -1, next = token_slot_of(P, t1, -1),
+                    prev = token_slot_of(P, t0, -1);
+      uint32_t w[8], w2[8];
+      float sc = 0.f, sc2 = 0.f;
+      row_codes<KV>(r[0], w, sc);
+      row_codes<KV>(r[1], w2, sc2);
+      const bool pair = (slot & 1) == 0 && more && next == slot + 1;
+      if (slot < 0 || i >= D / 8 || ((slot & 1) == 1 && n > 0 && prev == slot - 1)) return;
+      const int64_t tix = slot / BS * Hkv + h;
+      const int o = (int)(slot % BS);
+      uint8_t* L = base + (uint64_t)P.layer * P.g.layer_stride;
+      uint8_t* tile = L + P.g.v_off + (uint64_t)tix * P.g.tile_bytes;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        uint8_t* p = tile + tile_elem<true>(o & ~1, e ? b : a, ESZ, D);
+        if (pair) {
+          store4<ESZ>(p, w[4 * e], w2[4 * e], w[4 * e + 1], w2[4 * e + 1]);
+          store4<ESZ>(p + 4 * ESZ, w[4 * e + 2], w2[4 * e + 2], w[4 * e + 3], w2[4 * e + 3]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) store1<ESZ>(p + (2 * k + (o & 1)) * ESZ, w[4 * e + k]);
+        }
+      }
+      if (KV == KV_I8_REF && i == 0) {
+        float* s = reinterpret_cast<float*>(L + P.g.vs_off) + tix * BS + o;
+        s[0] = sc;
+        if (pair) s[1] = sc2;
       }
     }
     return;
   }
-  const bool is_v = (threadIdx.x >= WAVE);
-  uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
-  const void* src = is_v ? P.v : P.k;
-  uint8_t* codes = L + (is_v ? P.g.v_off : P.g.k_off);
-  if constexpr (KV == KV_I8_BLK) {
-    uint16_t* sc = reinterpret_cast<uint16_t*>(L + (is_v ? P.g.vs_off : P.g.ks_off));
-    if (is_v) append_blk<true, D>(P, src, codes, sc, w0, T); else append_blk<false, D>(P, src, codes, sc, w0, T);
-    return;
+  // RB query heads, the last ones clamped to the last head; K rows one by one.
+  const TokenIn tk_in = token_in(P, n);
+  Row8 r[RB];
+  int64_t rows[RB];
+#pragma unroll
+  for (int k = 0; k < RB; ++k) rows[k] = ((int64_t)n * nh + min(h + k, nh - 1)) * io;
+  load_rows8<RB>(src, dtype, rows, a, b, in, r);
+  bool rot = false;
+  float4 t0, t1;
+  if (P.rope != ROPE_NONE) {
+    const bool half = P.rope == ROPE_HALF;
+    const int pos = pos_of(P, tk_in);
+    rot = pos >= 0 && pos < P.n_pos;
+    const float* cs = P.cos_sin + (int64_t)(rot ? pos : 0) * io;
+    t0 = *reinterpret_cast<const float4*>(cs + (in ? (half ? 2 * a : a) : 0));
+    t1 = *reinterpret_cast<const float4*>(cs + (in ? (half ? 2 * a + 4 : b) : 0));
   }
-  // one token at a time; the window's slots are read at once (lane j: token w0 + j)
-  const int64_t ms = w0 + lane_id() < w1 ? token_slot(P, w0 + lane_id()) : -1;
-  for (int n = w0; n < w1; ++n) {
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)ms, n - w0);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)ms >> 32), n - w0);
-    const int64_t slot = (int64_t)(((uint64_t)hi << 32) | lo);
-    if constexpr (KV == KV_I8_REF) {
-      float* sc = reinterpret_cast<float*>(L + (is_v ? P.g.vs_off : P.g.ks_off));
-      if (is_v) append_ref<true>(P, src, codes, sc, n, slot); else append_ref<false>(P, src, codes, sc, n, slot);
-    } else if constexpr (KV == KV_F16) {
-      if (is_v) append_plain<true, 2>(P, src, codes, n, slot); else append_plain<false, 2>(P, src, codes, n, slot);
-    } else {
-      if (is_v) append_plain<true, 4>(P, src, codes, n, slot); else append_plain<false, 4>(P, src, codes, n, slot);
+  if (P.rope != ROPE_NONE) {
+    if (rot && in) {  // (the padding stays +0)
+#pragma unroll
+      for (int k = 0; k < RB; ++k) rope_row8(r[k], P.rope, t0, t1);
     }
   }
+  if (is_q) {  // unrotated rows stay as they are (copied when q_out is given)
+    if (!tok || !in || (!rot && !P.q_out)) return;
+    void* qd = P.q_out ? P.q_out : P.q;
+#pragma unroll
+    for (int e = 0; e < 2 * RB; ++e) {
+      if (RB > 1 && h + e / 2 >= nh) break;
+      const float* x = r[e / 2].x;
+      const int64_t o = (row + e / 2) * io + (e & 1 ? b : a);
+      if (dtype == DT_F16)
+        *reinterpret_cast<u32x2_in*>(reinterpret_cast<uint16_t*>(qd) + o) =
+            u32x2_in{(uint32_t)f2h(x[4 * (e & 1)]) | ((uint32_t)f2h(x[4 * (e & 1) + 1]) << 16),
+                     (uint32_t)f2h(x[4 * (e & 1) + 2]) | ((uint32_t)f2h(x[4 * (e & 1) + 3]) << 16)};
+      else
+        *reinterpret_cast<u32x4_in*>(reinterpret_cast<float*>(qd) + o) =
+            u32x4_in{__float_as_uint(x[4 * (e & 1)]), __float_as_uint(x[4 * (e & 1) + 1]), __float_as_uint(x[4 * (e & 1) + 2]),
+                     __float_as_uint(x[4 * (e & 1) + 3])};
+    }
+    return;
+  }
+  if constexpr (KV != KV_I8_BLK) {
+    uint32_t w[8];
+    float sc = 0.f;
+    row_codes<KV>(r[0], w, sc);
+    const int64_t slot = tok ? token_slot_of(P, tk_in, token_entry(P, n, tk_in)) : -1;
+    if (slot < 0 || i >= D / 8) return;
+    const int64_t t = slot / BS * Hkv + h;
+    const int o = (int)(slot % BS);
+    uint8_t* L = base + (uint64_t)P.layer * P.g.layer_stride;
+    uint8_t* tile = L + P.g.k_off + (uint64_t)t * P.g.tile_bytes;
+    store4<ESZ>(tile + tile_elem<false>(o, a, ESZ, D), w[0], w[1], w[2], w[3]);
+    store4<ESZ>(tile + tile_elem<false>(o, b, ESZ, D), w[4], w[5], w[6], w[7]);
+    if (KV == KV_I8_REF && i == 0) reinterpret_cast<float*>(L + P.g.ks_off)[t * BS + o] = sc;
+  }
+}
+
+// K row (wave 0) and V row (wave 1) of token n and KV head h: lane l holds dims 2l
+// and 2l + 1. The form of the calls whose workgroups are all resident at once
+// (kTokenWgs): bound by the chain from the arguments to the stores, which is shorter
+// than append_rows': 78 fp16 draft tokens x 8 heads 3.5 us against 4.0 in the kernel.
+template <int KV>
+DEV void append_token(const AppendParams& P, int n, int h) {
+  constexpr int ESZ = Esz<KV>::v;
+  const bool is_v = threadIdx.x >= WAVE;
+  const int64_t slot = token_slot(P, n);
+  if (slot < 0) return;
+  uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
+  const int64_t t = slot / BS * P.g.n_kv_heads + h;
+  const int o = (int)(slot % BS), d0 = 2 * lane_id(), D = P.g.head_dim;
+  float x0, x1;
+  load_kv(P, is_v ? P.v : P.k, is_v, n, h, x0, x1);
+  float inv = 0.f;
+  if constexpr (KV == KV_I8_REF) {
+    const float amax = wave_max(fmaxf(fabsf(x0), fabsf(x1)));
+    inv = amax > 0.f ? 127.0f / amax : 0.f;
+    if (d0 == 0) reinterpret_cast<float*>(L + (is_v ? P.g.vs_off : P.g.ks_off))[t * BS + o] = amax / 127.0f;
+  }
+  if (d0 >= D) return;
+  uint8_t* tile = L + (is_v ? P.g.v_off : P.g.k_off) + (uint64_t)t * P.g.tile_bytes;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    uint8_t* p = tile + (is_v ? tile_elem<true>(o, d0 + e, ESZ, D) : tile_elem<false>(o, d0 + e, ESZ, D));
+    const float x = e ? x1 : x0;
+    store1<ESZ>(p, ESZ == 1 ? (uint8_t)(int8_t)(int)(x * inv) : ESZ == 2 ? f2h(x) : __float_as_uint(x));
+  }
+}
+
+// Workgroups 0 .. kv_wgs - 1 take K and V of a KV head, heads fastest: the runs of a
+// window of tok_per_wg tokens (I8_BLK), or a token (small calls of the other types).
+// The others take a token group and a group of rows (append_rows), groups fastest.
+// D: head_dim of the pool for the I8_BLK rule (a compile-time constant, so that
+// the 16 tokens' tile offsets fold into the instructions; vk_append_kv3 / _d64).
+template <int KV, int D = HD>
+DEV void append_kernel(const AppendParams& P) {
+  if constexpr (KV == KV_I8_BLK) {
+    if ((int)blockIdx.x < P.kv_wgs) {
+      const int h = (int)blockIdx.x % P.g.n_kv_heads, w0 = (int)blockIdx.x / P.g.n_kv_heads * P.tok_per_wg;
+      uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
+      if (threadIdx.x >= WAVE)
+        append_blk<true, D>(P, P.v, L + P.g.v_off, reinterpret_cast<uint16_t*>(L + P.g.vs_off), w0, P.tok_per_wg, h);
+      else
+        append_blk<false, D>(P, P.k, L + P.g.k_off, reinterpret_cast<uint16_t*>(L + P.g.ks_off), w0, P.tok_per_wg, h);
+      return;
+    }
+  } else if ((int)blockIdx.x < P.kv_wgs) {
+    append_token<KV>(P, (int)blockIdx.x / P.g.n_kv_heads, (int)blockIdx.x % P.g.n_kv_heads);
+    return;
+  }
+  const int id = (int)blockIdx.x - P.kv_wgs;
+  append_rows<KV, row_batch(KV)>(P, id);
 }
 
 // =============================================================================

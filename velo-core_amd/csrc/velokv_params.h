@@ -50,10 +50,11 @@ enum RopeStyle : int32_t { ROPE_NONE = 0, ROPE_INTERLEAVED = 1, ROPE_HALF = 2 };
 // VK_MISUSE_*); the kernels still run to completion on the clamped input.
 enum Misuse : uint32_t { MISUSE_PAGE_OUT_OF_POOL = 1u, MISUSE_BLK_SPLIT_RUN = 2u };
 
-// Append of n_tok tokens; grid (ceil(n_tok / tok_per_wg), Hkv + ceil(n_heads / 2)):
-// workgroup x covers tokens [x T, x T + T) of the call, T = tok_per_wg; rows
-// y < Hkv write K (wave 0) and V (wave 1) of KV head y; with RoPE, rows y >= Hkv
-// rotate query heads 2(y - Hkv) and 2(y - Hkv) + 1 in place.
+// Append of n_tok tokens, workgroups of two waves: kv_wgs = ceil(n_tok / T) Hkv of
+// them (I8_BLK pools, else 0; T = tok_per_wg) write K (wave 0) and V (wave 1) of a
+// KV head and the runs that start in a window of T tokens; ceil(n_tok / 8)
+// row_groups follow for the rows that are stored one by one: query heads to
+// rotate, and K and V of the other pool types.
 struct AppendParams {
   uint8_t* base;            // pool base (all layers)
   PoolGeom g;
@@ -71,7 +72,9 @@ struct AppendParams {
   void* q;                  // [n_tok][n_heads][D] of q_dtype, rotated in place unless q_out is given
   void* q_out;              // or the rotated rows go here (same shape and type), q left unchanged
   int32_t q_dtype;
-  int32_t tok_per_wg;       // tokens per workgroup (1..64)
+  int32_t tok_per_wg;       // I8_BLK: tokens per workgroup (1..64)
+  int32_t kv_wgs;           // workgroups of the I8_BLK runs, or of a token and KV head each (small calls)
+  int32_t row_groups;       // row groups per token: query heads, row_batch of them each; K and V heads (not I8_BLK)
   uint32_t* err;            // the context's misuse word
   unsigned long long* claim;// I8_BLK: [n_blocks] (epoch << 32 | first token) of the last run per block
   uint32_t epoch;           // I8_BLK: this call's epoch (never 0)
@@ -81,7 +84,15 @@ struct AppendParams {
   const int32_t* seq_rows;
   const int32_t* context_lens;
   int32_t bt_stride, bt_rows, cap_tokens;
+  // slot_mapping, positions and context_lens, or where there is none a word that
+  // exists (the kernels load it with no branch and ignore it)
+  const int64_t* slot_any;
+  const int32_t *pos_any, *ctx_any;
 };
+
+// Query heads per row group: more where the kernel's registers (the I8_BLK rule's)
+// hold fewer waves.
+constexpr int row_batch(int kv_type) { return kv_type == KV_I8_BLK ? 4 : 2; }
 
 struct SlotMapParams {
   const int32_t* block_tables;
@@ -117,7 +128,7 @@ struct DecodeParams {
   int32_t page_tiles;       // page tokens / 16: table entry p holds tiles p * page_tiles .. (p + 1) * page_tiles - 1
   int32_t io_hd;            // head_dim: q / out row length (a multiple of 8 up to 128)
   int32_t tile_hd;          // tile width, 64 or 128 (>= io_hd; the dims past io_hd hold zeros)
-  int32_t max_parts;        // partitions per sequence in the grid (workgroup split: at most)
+  int32_t max_parts;        // partitions per sequence in the grid
   int32_t part_tokens;      // tokens per partition (multiple of the block size)
   int32_t cap_tokens;       // tokens a table row can address: min(max_parts*part_tokens, bt_stride*bs)
   int32_t n_nodes;          // query rows per (sequence, head): 1 for decode
@@ -131,7 +142,8 @@ struct DecodeParams {
   // the prefix pass, the partitions of the rest of the context follow
   int32_t prefix_blocks, prefix_chunks;
   uint32_t* err;            // the context's misuse word (page ids outside the pool)
-  // vk_append_decode with the append folded into the decode (null otherwise): the new K and V rows [n_seqs][n_kv_heads][io_hd] of
+  // vk_append_decode over an I8_BLK pool with the append folded into the decode
+  // (null otherwise): the new K and V rows [n_seqs][n_kv_heads][io_hd] of
   // fold_dtype, the call's append epoch and the pool's per-tile claim words
   const void* fold_k;
   const void* fold_v;
