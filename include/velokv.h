@@ -450,7 +450,8 @@ typedef struct vk_tree_args {
 } vk_tree_args;
 
 /* Bytes of split-K workspace vk_tree_verify needs for these arguments (0 when
- * one partition covers every sequence). */
+ * one partition covers every sequence). Calls of few units take partitions of less
+ * than 256 tokens; with a smaller buffer, which 256-token ones fit, they take those. */
 int vk_tree_verify_workspace(const vk_pool* pool, const vk_tree_args* a, uint64_t* bytes);
 
 /* What vk_tree_verify would launch for these arguments, launching nothing. No

@@ -1311,7 +1311,13 @@ struct TreePlan {
   std::string kernel, pfx_kernel;
 };
 
-int plan_tree(vk_ctx* ctx, const vk_pool* pool, const vk_tree_args* a, TreePlan* pl) {
+// The least partitions of a tree call of few units, in tokens, and the waves per CU
+// up to which they are taken (plan_tree).
+constexpr int kTreeShort[] = {64, 96, 128, 192};
+constexpr int64_t kTreeShortWaves = 4;
+
+// short_parts: partitions of less than 256 tokens may be taken (they need more scratch).
+int plan_tree(vk_ctx* ctx, const vk_pool* pool, const vk_tree_args* a, TreePlan* pl, bool short_parts = true) {
   if (!a) return fail(VK_ERR_BAD_ARG, "args is null");
   const vk_pool_desc& d = pool->desc;
   if (a->layer < 0 || a->layer >= d.n_layer) return fail(VK_ERR_BAD_ARG, "layer %d out of range", a->layer);
@@ -1383,6 +1389,19 @@ int plan_tree(vk_ctx* ctx, const vk_pool* pool, const vk_tree_args* a, TreePlan*
     P = kMaxPartTokens;
     for (int c = 256; c < kMaxPartTokens; c *= 2)
       if (pairs * ((tokens + c - 1) / c) <= 4 * waves) { P = c; break; }
+    // Calls whose units leave SIMDs empty take shorter ones, the shortest whose
+    // units are at most one wave per SIMD: a wave walks its blocks one after
+    // another (about 1.2 us a block over fp16, 2.6 over fp32), and past one wave
+    // per SIMD the merge and its partials cost more than the walk saves. 64 / 256
+    // tokens at 8 nodes: 1,500 int8 tokens, 4 units a partition, 9.7 / 15.1 us;
+    // 4,000 fp32 tokens, 16 units, 18.6 / 33.7. Past the line, 192 / 256: 512 units
+    // a partition, 4,000 int8 tokens, 99.8 / 95.3; 192 units, 1,500 fp16 tokens,
+    // 44.0 / 32.1. A call that one 256-token partition covers stays whole: it needs
+    // no scratch, so such calls on several streams share nothing.
+    const int64_t simds = std::min(waves, kTreeShortWaves * (ctx ? ctx->n_cu : 256));
+    if (short_parts && P == 256 && tokens > 256 && pl->prefix_chunks == 0)
+      for (int c : kTreeShort)
+        if (pairs * ((tokens + c - 1) / c) <= simds) { P = c; break; }
   }
   pl->part_tokens = P;
   pl->max_parts = pl->prefix_chunks + (int32_t)std::max<int64_t>(1, (tokens + P - 1) / P);
@@ -1422,6 +1441,21 @@ extern "C" int vk_tree_verify_plan(const vk_pool* pool, const vk_tree_args* a, v
   return VK_OK;
 }
 
+namespace {
+// Whether a call can have `need` bytes of scratch: in the caller's buffer, or in
+// the context's own, which may grow unless the stream is being captured.
+bool tree_scratch_at_hand(vk_ctx* ctx, const vk_tree_args* a, uint64_t need, void* stream) {
+  if (a->workspace) return a->workspace_bytes >= need;
+  {
+    std::lock_guard<std::mutex> lk(ctx->ws_mu);
+    if (ctx->ws_bytes >= need) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return !stream || (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &st) == hipSuccess &&
+                     st == hipStreamCaptureStatusNone);
+}
+}  // namespace
+
 extern "C" int vk_tree_verify(vk_ctx* ctx, vk_pool* pool, const vk_tree_args* a, void* stream) {
   int rc = check_pool(ctx, pool);
   if (rc) return rc;
@@ -1430,6 +1464,11 @@ extern "C" int vk_tree_verify(vk_ctx* ctx, vk_pool* pool, const vk_tree_args* a,
   if (a->n_seqs == 0) return VK_OK;
   if (!a->q || !a->out || !a->context_lens || !a->tree_mask) return fail(VK_ERR_BAD_ARG, "null device pointer");
   if ((rc = set_device(ctx))) return rc;
+  // short partitions only where their scratch is at hand: not past the caller's
+  // buffer, and no growing of the context's own under capture
+  if (pl.max_parts > 1 && !tree_scratch_at_hand(ctx, a, pl.acc_bytes + pl.ml_bytes, stream) &&
+      (rc = plan_tree(ctx, pool, a, &pl, false)))
+    return rc;
   uint8_t* ws = nullptr;
   if (pl.max_parts > 1 &&
       (rc = split_workspace(ctx, a->workspace, a->workspace_bytes, pl.acc_bytes + pl.ml_bytes, &ws)))
