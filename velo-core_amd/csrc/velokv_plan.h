@@ -1,0 +1,87 @@
+// Rules that choose a decode plan from a call's sizes alone: host code with no HIP
+// in it, so that a host test can sweep them.
+#pragma once
+#include "velokv.h"
+
+#include <algorithm>
+#include <cstdint>
+
+namespace velokv {
+
+constexpr int kBS = 16;   // tokens per tile, the kernels' block
+constexpr int kMaxPartTokens = 4096;  // 256 blocks: four block-id windows of one wave
+constexpr int kWgMaxWaves = 8;  // waves per workgroup of vk_decode_wg_* / vk_decode_pk_* at most (velokv_kernels.hip)
+
+inline int kv_esz(int kv) {
+  switch (kv) {
+    case VK_KV_F32: return 4;
+    case VK_KV_F16: return 2;
+    case VK_KV_I8_REF:
+    case VK_KV_I8_BLK: return 1;
+    default: return 0;
+  }
+}
+
+// Small batches under VK_SCHED_AUTO take the workgroup split in one or a few
+// partitions per sequence (small_plan) while their (sequence, KV head) pairs
+// have at most this many blocks in all: ragged batches; uniform ones; uniform
+// ones over fp16 pools or of at most kFewPairs pairs, where the alternative is
+// split-K of one-wave units.
+constexpr int64_t kSmallRagged = 16384;
+constexpr int64_t kSmallUniform = 12288;
+constexpr int64_t kSmallUniformWide = 65536;
+constexpr int64_t kFewPairs = 64;
+// K and V bytes of the least partition worth a workgroup, and of what a
+// partition must take off the longest context's workgroup to pay for the merge
+// launch it brings (3.4 us; a workgroup alone on its CU streams 43 KB per us).
+constexpr int64_t kMinPartBytes = 65536;
+constexpr int64_t kMergeBytes = 147456;
+// Workgroups of a call in partitions at most: bounds the scratch (17 MB at 16
+// query heads per KV head) and the workgroups past short contexts.
+constexpr int64_t kMaxPartWgs = 2048;
+
+inline bool uniform_batch(const vk_decode_args* a) {
+  return a->sum_context_len > 0 &&
+         (double)a->sum_context_len >= 0.97 * (double)a->n_seqs * (double)a->max_context_len;
+}
+
+// Workgroup split of a small batch (VK_SCHED_AUTO): *waves waves per (sequence,
+// partition of *part_blocks blocks, KV head); false when the batch is too large
+// for it. waves_total: resident waves of the kernel; tile: K bytes of one block
+// and KV head. The lengths' sum only steers the choice: any lengths up to
+// max_context_len are computed whatever it says.
+inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves_total, int64_t tile, int* waves,
+                       int64_t* part_blocks) {
+  const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
+  const int64_t pairs = (int64_t)a->n_seqs * d.n_kv_heads;
+  if (pairs <= 0 || nb <= 0 || pairs > waves_total) return false;
+  // lengths the host does not know (any up to max_context_len) stay with stream-K,
+  // which balances whatever they are
+  if (a->sum_context_len <= 0 && a->n_seqs > 1) return false;
+  // blocks of one KV head over all sequences (at most, when the lengths are not known)
+  const int64_t most = (int64_t)a->n_seqs * nb;
+  const int64_t sum = a->sum_context_len > 0 ? std::min(most, a->sum_context_len / kBS + a->n_seqs) : most;
+  int64_t limit = kSmallRagged;
+  if (uniform_batch(a)) limit = d.kv_type == VK_KV_F16 || pairs <= kFewPairs ? kSmallUniformWide : kSmallUniform;
+  if (sum * d.n_kv_heads > limit) return false;
+  // uniform contexts of up to four int8 blocks (one fp32 block) take one wave of
+  // split-K, whose result needs no combining (5.6 us per call at two int8 blocks;
+  // fp16 split-K runs the vector kernel, 13.0 us at 16 x 32 tokens against 5.6)
+  if (uniform_batch(a) && d.kv_type != VK_KV_F16 && nb * kv_esz(d.kv_type) <= 4) return false;
+  int nw = nb <= kWgMaxWaves ? kWgMaxWaves / 2 : kWgMaxWaves;
+  while (nw > 1 && pairs * nw > waves_total) nw /= 2;
+  *waves = nw;
+  *part_blocks = nb;
+  if (nw < kWgMaxWaves) return true;
+  // partitions whose workgroups fit one round: at most floor(slots / S) per
+  // sequence, or sum / part + S in all (a partial one per sequence)
+  const int64_t slots = waves_total / kWgMaxWaves / d.n_kv_heads;
+  const int64_t per = std::max<int64_t>(1, slots / a->n_seqs);
+  int64_t part = (nb + per - 1) / per;
+  if (slots > a->n_seqs) part = std::min(part, (sum + slots - a->n_seqs - 1) / (slots - a->n_seqs));
+  part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
+  if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
+  return true;
+}
+
+}  // namespace velokv
