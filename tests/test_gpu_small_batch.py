@@ -134,3 +134,31 @@ def test_append_of_one_sequence_twice(ctx, kv):
     ctx.sync()
     assert_layer_equal(pool, 0, ref)
     close(out.download(q.shape, np.float32), O.paged_decode(ref, q, bt, lens), kv, np.float16)
+
+
+# one long context among many short ones: KV heads, lengths
+SKEWED = [(8, [20000] + [200] * 39), (8, [10000] + [150] * 69), (8, [5000] + [60] * 199), (2, [40000] + [200] * 99)]
+
+
+@pytest.mark.parametrize("shape", range(len(SKEWED)))
+def test_skewed_batch(ctx, shape):
+    """Every wave's range within the 256 blocks it can hold, and the append and the outputs right."""
+    hkv, lens = SKEWED[shape]
+    case = make_case(O.F16, lens, n_kv_heads=hkv, n_heads=hkv, seed=3500 + shape)
+    q, cl, tab = ctx.upload(case.q), ctx.upload(case.ctx_lens), ctx.upload(case.block_tables)
+    _, kk, vv = case.last_slots()
+    for kv in (O.F32, O.F16, O.I8_REF, O.I8_BLK):
+        print(f"small skewed kv={kv} {hkv} heads, {len(lens)} sequences, longest {lens[0]}", flush=True)
+        case.kv_type = kv
+        pool = gpu_pool(ctx, case, with_last=False)
+        for total in (sum(lens), 7):
+            pl = plan(ctx, pool, case, np.float16, total)
+            assert pl["max_blocks_per_wave"] <= 256, pl
+        out = ctx.alloc(case.q.size * 4)
+        ctx.append_decode(pool, 0, ctx.upload(kk), ctx.upload(vv), velokv.DT_F16, q, velokv.DT_F16, out, cl, case.S, hkv,
+                          lens[0], block_tables=tab, bt_stride=case.block_tables.shape[1], sum_context_len=sum(lens))
+        ctx.sync()
+        ref = oracle_layer_in(case, np.float16)
+        assert_layer_equal(pool, 0, ref)
+        want = O.paged_decode(ref, case.q, case.block_tables, case.ctx_lens)
+        close(out.download(case.q.shape, np.float32), want, kv, np.float16)

@@ -47,7 +47,7 @@ inline bool uniform_batch(const vk_decode_args* a) {
 
 // Workgroup split of a small batch (VK_SCHED_AUTO): *waves waves per (sequence,
 // partition of *part_blocks blocks, KV head); false when the batch is too large
-// for it. waves_total: resident waves of the kernel; tile: K bytes of one block
+// for it, or a wave's share of its longest context is. waves_total: resident waves of the kernel; tile: K bytes of one block
 // and KV head. The lengths' sum only steers the choice: any lengths up to
 // max_context_len are computed whatever it says.
 inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves_total, int64_t tile, int* waves,
@@ -72,16 +72,19 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t w
   while (nw > 1 && pairs * nw > waves_total) nw /= 2;
   *waves = nw;
   *part_blocks = nb;
-  if (nw < kWgMaxWaves) return true;
-  // partitions whose workgroups fit one round: at most floor(slots / S) per
-  // sequence, or sum / part + S in all (a partial one per sequence)
-  const int64_t slots = waves_total / kWgMaxWaves / d.n_kv_heads;
-  const int64_t per = std::max<int64_t>(1, slots / a->n_seqs);
-  int64_t part = (nb + per - 1) / per;
-  if (slots > a->n_seqs) part = std::min(part, (sum + slots - a->n_seqs - 1) / (slots - a->n_seqs));
-  part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
-  if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
-  return true;
+  if (nw == kWgMaxWaves) {
+    // partitions whose workgroups fit one round: at most floor(slots / S) per
+    // sequence, or sum / part + S in all (a partial one per sequence)
+    const int64_t slots = waves_total / kWgMaxWaves / d.n_kv_heads;
+    const int64_t per = std::max<int64_t>(1, slots / a->n_seqs);
+    int64_t part = (nb + per - 1) / per;
+    if (slots > a->n_seqs) part = std::min(part, (sum + slots - a->n_seqs - 1) / (slots - a->n_seqs));
+    part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
+    if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
+  }
+  // a wave holds the ids of 256 blocks (four windows): the longest context the call
+  // allows must fit, whatever the sum says, as every other plan sees to
+  return (*part_blocks + nw - 1) / nw <= kMaxPartTokens / kBS;
 }
 
 }  // namespace velokv
