@@ -31,7 +31,41 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
            (long long)longest, (long long)sum, kv, dim, (long long)resident, waves, (long long)part);
 }
 
+// One sequence of `longest` tokens and n - 1 of `rest`, 2,048 resident waves: whether the rule
+// takes the batch (measured both ways: us of the small plan, of stream-K).
+struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; };
+static const Skewed kSkewed[] = {
+    {VK_KV_I8_BLK, 8, 64, 500, 200, true, 12.3, 18.9},   {VK_KV_I8_BLK, 8, 64, 16000, 200, false, 122.3, 33.6},
+    {VK_KV_I8_BLK, 8, 128, 4000, 100, false, 67.2, 23.4}, {VK_KV_I8_BLK, 8, 16, 8000, 500, true, 17.1, 29.6},
+    {VK_KV_I8_BLK, 2, 100, 16000, 200, false, 100.3, 52.5}, {VK_KV_I8_BLK, 2, 40, 4000, 200, true, 13.6, 39.0},
+    {VK_KV_F16, 8, 33, 2000, 200, false, 31.8, 20.1},    {VK_KV_F16, 4, 64, 4000, 200, false, 53.7, 24.0},
+    {VK_KV_F16, 8, 24, 500, 300, true, 10.5, 16.0},      {VK_KV_F16, 2, 100, 8000, 200, true, 21.3, 36.0},
+    {VK_KV_I8_REF, 8, 40, 8000, 200, false, 67.7, 30.4}, {VK_KV_I8_REF, 8, 24, 8000, 300, true, 24.8, 31.1},
+    {VK_KV_F32, 8, 24, 16000, 300, false, 84.4, 65.2},   {VK_KV_F32, 8, 16, 16000, 500, true, 54.9, 65.3},
+    {VK_KV_F32, 8, 200, 2000, 60, false, 211.2, 50.0},   {VK_KV_F32, 8, 24, 500, 300, true, 24.4, 32.3},
+    {VK_KV_F16, 4, 199, 335, 180, true, 12.8, 16.9},
+};
+
+static void check_skewed(const Skewed& c) {
+  vk_decode_args a;
+  vk_pool_desc d;
+  memset(&a, 0, sizeof a);
+  memset(&d, 0, sizeof d);
+  a.n_seqs = c.n;
+  a.max_context_len = c.longest;
+  a.sum_context_len = c.longest + (int64_t)(c.n - 1) * c.rest;
+  d.n_kv_heads = c.hkv;
+  d.kv_type = c.kv;
+  int waves = 0;
+  int64_t part = 0;
+  if (small_plan(&a, d, 2048, (int64_t)kBS * 128 * kv_esz(c.kv), &waves, &part) == c.small) return;
+  if (bad++ < 10)
+    printf("skewed: kv %d, %d x %d heads, longest %d, rest %d: small %d (%.1f us, stream-K %.1f)\n", c.kv, c.n, c.hkv,
+           c.longest, c.rest, !c.small, c.us, c.sk_us);
+}
+
 int main() {
+  for (const Skewed& c : kSkewed) check_skewed(c);
   for (int64_t resident : {1024, 2048, 4096, 8192})
     for (int kv : {VK_KV_F32, VK_KV_F16, VK_KV_I8_REF, VK_KV_I8_BLK})
       for (int dim : {64, 128})

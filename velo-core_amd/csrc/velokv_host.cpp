@@ -742,11 +742,6 @@ int split_workspace(vk_ctx* ctx, void* given, uint64_t given_bytes, uint64_t nee
 constexpr int kPkMaxSeqs = 256;  // sequences a vk_decode_pk_* workgroup ranks
 constexpr int kPkMaxRounds = 16; // items per vk_decode_pk_* workgroup
 
-// Stream-K cost units charged to each segment ahead of its blocks, for what a
-// worker spends starting a second piece (per-wave traces on config 3: ~5 us).
-// Measured on configs 2 and 3 with 0, 4, 8, 12, 16, 24: 8 was fastest (config 3
-// 110.7 -> 109.2 us per call, config 2 208 -> 206 us).
-constexpr int kSkPenalty = 8;
 // Blocks' worth of time the append costs the wave that folds it into a
 // workgroup-split decode (vk_append_decode over I8_BLK pools): that wave's range
 // is this much shorter.

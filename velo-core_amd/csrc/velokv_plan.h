@@ -12,6 +12,12 @@ constexpr int kBS = 16;   // tokens per tile, the kernels' block
 constexpr int kMaxPartTokens = 4096;  // 256 blocks: four block-id windows of one wave
 constexpr int kWgMaxWaves = 8;  // waves per workgroup of vk_decode_wg_* / vk_decode_pk_* at most (velokv_kernels.hip)
 
+// Stream-K cost units charged to each segment ahead of its blocks, for what a
+// worker spends starting a second piece (per-wave traces on config 3: ~5 us).
+// Measured on configs 2 and 3 with 0, 4, 8, 12, 16, 24: 8 was fastest (config 3
+// 110.7 -> 109.2 us per call, config 2 208 -> 206 us).
+constexpr int kSkPenalty = 8;
+
 inline int kv_esz(int kv) {
   switch (kv) {
     case VK_KV_F32: return 4;
@@ -39,6 +45,19 @@ constexpr int64_t kMergeBytes = 147456;
 // Workgroups of a call in partitions at most: bounds the scratch (17 MB at 16
 // query heads per KV head) and the workgroups past short contexts.
 constexpr int64_t kMaxPartWgs = 2048;
+// A ragged batch stays with stream-K when its longest context keeps one wave busy
+// for longer than the small plan saves: bytes per us of a wave among eight of a
+// workgroup, and among fewer; the merge launch of partitions; what stream-K costs
+// beside its blocks, and for each partial that it leaves of the longest context
+// (its merge reads them in turn). In ns. Fitted to 319 ragged batches, skewed ones (16 to 200
+// sequences, one of 500 to 16,000 tokens and the others of 60 to 500) and evenly
+// spread ones, four KV types:
+// 64 x 8 heads of 200 int8-block tokens, one of 1,000 15.4 us against stream-K's 19.1,
+// one of 2,000 22.1 against 20.2, one of 16,000 122 against 33.6; fp16 one of 500 16.3
+// against 19.8, one of 1,000 22.4 against 20.2.
+constexpr int64_t kWaveRate8 = 5400, kWaveRate = 9000;
+constexpr int64_t kMergeNs = 3400;
+constexpr int64_t kSkFixedNs = 9000, kSkPartialNs = 80;
 
 inline bool uniform_batch(const vk_decode_args* a) {
   return a->sum_context_len > 0 &&
@@ -47,8 +66,8 @@ inline bool uniform_batch(const vk_decode_args* a) {
 
 // Workgroup split of a small batch (VK_SCHED_AUTO): *waves waves per (sequence,
 // partition of *part_blocks blocks, KV head); false when the batch is too large
-// for it, or a wave's share of its longest context is. waves_total: resident waves of the kernel; tile: K bytes of one block
-// and KV head. The lengths' sum only steers the choice: any lengths up to
+// for it, or a wave's share of its longest context is. waves_total: resident waves
+// of the kernel; tile: K bytes of one block and KV head. The lengths' sum only steers the choice: any lengths up to
 // max_context_len are computed whatever it says.
 inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves_total, int64_t tile, int* waves,
                        int64_t* part_blocks) {
@@ -81,6 +100,14 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t w
     if (slots > a->n_seqs) part = std::min(part, (sum + slots - a->n_seqs - 1) / (slots - a->n_seqs));
     part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
     if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
+  }
+  if (!uniform_batch(a) && a->n_seqs > 1) {
+    const int64_t even = sum * d.n_kv_heads * 2 * tile / waves_total;  // bytes of a wave if all had the same
+    const int64_t wave = (*part_blocks + nw - 1) / nw * 2 * tile;
+    const int64_t late = std::max<int64_t>(0, wave - even) * 1000 / (nw == kWgMaxWaves ? kWaveRate8 : kWaveRate) +
+                         (*part_blocks < nb ? kMergeNs : 0);
+    const int64_t share = std::max<int64_t>(1, (sum * d.n_kv_heads + kSkPenalty * pairs) / waves_total);
+    if (late > kSkFixedNs + kSkPartialNs * (nb / share)) return false;
   }
   // a wave holds the ids of 256 blocks (four windows): the longest context the call
   // allows must fit, whatever the sum says, as every other plan sees to
