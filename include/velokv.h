@@ -373,10 +373,10 @@ int vk_paged_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* s
  * VK_MISUSE_PAGE_OUT_OF_POOL). The pool afterwards equals vk_append of those
  * slots followed by vk_paged_decode, bit for bit, and so do the outputs except
  * under the workgroup split, whose folding wave takes a few blocks fewer (the
- * outputs then agree to fp32 rounding of a different split). Over VK_KV_I8_BLK pools under the
- * workgroup-split or stream-K schedule, over VK_KV_F16 pools for ragged batches under
- * either, and over any pool for one sequence under the workgroup split, the decode
- * launch appends the tokens itself (the
+ * outputs then agree to fp32 rounding of a different split). Over VK_KV_I8_BLK pools under stream-K
+ * and under a workgroup split of ragged batches or of uniform ones that fill the GPU,
+ * over VK_KV_F16 pools for ragged batches under either, and over any pool for one
+ * sequence under the workgroup split, the decode launch appends the tokens itself (the
  * wave that holds a sequence's last block applies the append rule to it before
  * loading it; two sequences whose new tokens share a block are reported,
  * VK_MISUSE_BLK_SPLIT_RUN); otherwise the append kernel runs first, with the

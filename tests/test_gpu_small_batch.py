@@ -113,23 +113,27 @@ def test_append(ctx, kv, style, lens):
         close(out.download(case.q.shape, np.float32), want, kv, qd)
 
 
-@pytest.mark.parametrize("kv", [O.F32, O.F16, O.I8_REF])
-def test_append_of_one_sequence_twice(ctx, kv):
+@pytest.mark.parametrize("first", [200, 208])  # the two tokens in one block, in two
+@pytest.mark.parametrize("kv", [O.F32, O.F16, O.I8_REF, O.I8_BLK])
+def test_append_of_one_sequence_twice(ctx, kv, first):
     """Two rows of the call on one table row at lengths L and L + 1: both tokens are stored before
     either row attends, so the second sees the first (uniform batches keep the append launch)."""
-    print(f"small append of one sequence twice kv={kv}", flush=True)
-    case = make_case(kv, [200], n_kv_heads=2, n_heads=8, seed=3400)
+    print(f"small append of one sequence twice kv={kv} first={first}", flush=True)
+    case = make_case(kv, [first], n_kv_heads=2, n_heads=8, seed=3400)
     pool = gpu_pool(ctx, case, with_last=False)
     r = np.random.default_rng(3401)
     k, v = (r.standard_normal((2, 2, 128)).astype(np.float16) for _ in range(2))
     q = r.standard_normal((2, 8, 128)).astype(np.float16)
-    lens = np.array([200, 201], np.int32)
-    bt = np.repeat(case.block_tables, 2, 0)
+    lens = np.array([first, first + 1], np.int32)
+    bt = np.zeros((2, first // BS + 1), np.int32)
+    bt[:, :case.block_tables.shape[1]] = case.block_tables
+    if first % BS == 0:
+        bt[:, -1] = next(b for b in range(case.n_blocks) if b not in case.block_tables)
     ref = oracle_layer(case, with_last=False)
     O.append(ref, k, v, np.array([bt[0, (n - 1) // BS] * BS + (n - 1) % BS for n in lens], np.int64))
     out = ctx.alloc(q.size * 4)
     ctx.append_decode(pool, 0, ctx.upload(k), ctx.upload(v), velokv.DT_F16, ctx.upload(q), velokv.DT_F16, out,
-                      ctx.upload(lens), 2, 8, 201, block_tables=ctx.upload(bt), bt_stride=bt.shape[1],
+                      ctx.upload(lens), 2, 8, first + 1, block_tables=ctx.upload(bt), bt_stride=bt.shape[1],
                       sum_context_len=int(lens.sum()))
     ctx.sync()
     assert_layer_equal(pool, 0, ref)

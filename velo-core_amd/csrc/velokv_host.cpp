@@ -757,6 +757,7 @@ struct DecodePlan {
   int32_t n_workers;
   int32_t wg_waves;  // > 0: workgroup-split kernel with this many waves per (sequence, KV head)
   int32_t max_wave_blocks;  // packed: bound on the blocks of one wave's range
+  bool fills;        // workgroup split of a uniform batch whose workgroups fill the GPU (wg_fills)
   std::string kernel;
   uint64_t acc_bytes, ml_bytes, prefix_bytes;
 };
@@ -793,6 +794,17 @@ int auto_partition(const vk_decode_args* a, const vk_pool_desc& d, int64_t resid
   return kMaxPartTokens;
 }
 
+// Workgroup split of a uniform batch: the smallest power of two of waves per
+// (sequence, KV head) whose workgroups fill one round of resident waves, when each
+// wave's share fits its four block-id windows (256 blocks); 0 when none does.
+int wg_fills(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves) {
+  const int64_t pairs = (int64_t)a->n_seqs * d.n_kv_heads;
+  int nw = 1;
+  while (nw < 8 && pairs * nw < waves) nw *= 2;
+  const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
+  return pairs > 0 && pairs * nw >= waves && (nb + nw - 1) / nw <= kMaxPartTokens / kBS && pairs <= 0x7FFFFFFF ? nw : 0;
+}
+
 int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, DecodePlan* pl) {
   if (!a) return fail(VK_ERR_BAD_ARG, "args is null");
   const vk_pool_desc& d = pool->desc;
@@ -825,17 +837,20 @@ int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, Decod
   pl->wg_waves = 0;
   pl->packed = false;
   pl->max_wave_blocks = 0;
+  pl->fills = false;
   const int sched = ctx ? ctx->decode_sched : VK_SCHED_AUTO;
   // (VK_DECODE_VALU asks for the vector kernels of fixed partitions)
   const bool valu = ctx && ctx->decode_kind == VK_DECODE_VALU && fixed_group(G) && d.head_dim == kHD;
   int64_t part = 0;
   int waves = 0;
   const std::string wg = decode_wg_name(d.kv_type, G, a->q_dtype, d64);
+  const int64_t wg_waves = ctx ? resident_waves(ctx, wg, 64 * kWgMaxWaves) : 2048;
   if (sched == VK_SCHED_AUTO && !valu && P == 0 && G <= kMaxGroupTile &&
-      small_plan(a, d, ctx ? resident_waves(ctx, wg, 64 * kWgMaxWaves) : 2048, pool->geom.tile_bytes, &waves, &part)) {
+      small_plan(a, d, wg_waves, pool->geom.tile_bytes, &waves, &part)) {
     const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
     pl->stream_k = false;
     pl->wg_waves = waves;
+    pl->fills = wg_fills(a, d, wg_waves) != 0;
     pl->kernel = wg;
     pl->part_tokens = (int32_t)part * kBS;
     pl->max_parts = (int32_t)((nb + part - 1) / part);
@@ -893,18 +908,10 @@ int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, Decod
   // (fp16 pools at 128 dims: the dot2 split-K, or the matrix-core split-K with an
   // fp32 q, measured faster than a workgroup split; at 64 dims the split wins)
   if (mfma && P == 0 && G <= kMaxGroupTile && (d.kv_type != VK_KV_F16 || d64)) {
-    // Workgroup split: NW waves per (sequence, KV head), the smallest power of two
-    // whose workgroups fill one round of resident waves, when each wave's share
-    // fits its four block-id windows (256 blocks).
-    const int64_t pairs = (int64_t)a->n_seqs * d.n_kv_heads;
-    const int64_t waves = ctx ? resident_waves(ctx, decode_wg_name(d.kv_type, G, a->q_dtype, d64), 64 * kWgMaxWaves) : 2048;
-    int nw = 1;
-    while (nw < 8 && pairs * nw < waves) nw *= 2;
-    const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
-    if (pairs > 0 && pairs * nw >= waves && (nb + nw - 1) / nw <= kMaxPartTokens / kBS &&
-        pairs <= 0x7FFFFFFF) {
+    if (const int nw = wg_fills(a, d, wg_waves)) {
       pl->wg_waves = nw;
-      pl->kernel = decode_wg_name(d.kv_type, G, a->q_dtype, d64);
+      pl->fills = true;
+      pl->kernel = wg;
       pl->part_tokens = kMaxPartTokens;
       pl->max_parts = 1;
       return VK_OK;
@@ -985,13 +992,17 @@ namespace {
 // appended at position context_len - 1 of its table row by the append kernel,
 // slots derived in the kernel (the unfused half of vk_append_decode).
 // Whether the decode launch of this plan appends the new tokens itself
-// (vk_append_decode): I8_BLK pools under the workgroup split or stream-K, fp16
-// pools under stream-K, over tiles the folded kernels are built for.
+// (vk_append_decode), over tiles the folded kernels are built for: I8_BLK pools
+// under stream-K and under a workgroup split of ragged batches or of uniform ones
+// that fill the GPU, fp16 pools for ragged batches under either, any pool for one
+// sequence under the workgroup split. The others keep the append launch: a call may
+// list one sequence at two lengths, and the longer row must see the shorter one's
+// token, which no order between the workgroups of one launch gives.
 bool plan_folds_append(const vk_pool* pool, const vk_decode_args* a, const DecodePlan& pl) {
   const int kvt = pool->desc.kv_type;
-  const bool alone = a->n_seqs == 1 && pl.wg_waves > 0;
-  return ((kvt == VK_KV_I8_BLK && (pl.wg_waves > 0 || pl.stream_k)) ||
-          (kvt == VK_KV_F16 && (pl.stream_k || (pl.wg_waves > 0 && !uniform_batch(a)))) || alone) &&
+  const bool wg = pl.wg_waves > 0, ragged = !uniform_batch(a);
+  return ((kvt == VK_KV_I8_BLK && (pl.stream_k || (wg && (ragged || pl.fills)))) ||
+          (kvt == VK_KV_F16 && (pl.stream_k || (wg && ragged))) || (wg && a->n_seqs == 1)) &&
          (tile_hd(pool->desc.head_dim) == kHD || use_d64(pool->desc, a->n_heads / pool->desc.n_kv_heads));
 }
 
@@ -1056,10 +1067,9 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
   if (a->n_seqs == 0) return VK_OK;
   if (!a->q || !a->out || !a->context_lens) return fail(VK_ERR_BAD_ARG, "null device pointer");
   if ((rc = set_device(ctx))) return rc;
-  // I8_BLK pools under the workgroup split or stream-K, and fp16 pools under
-  // stream-K, take the append inside the decode launch (the wave that holds a
-  // sequence's last block appends the token before loading it); every other
-  // plan appends in a launch of its own first
+  // plan_folds_append: the append inside the decode launch (the wave that holds a
+  // sequence's last block appends the token before loading it); every other plan
+  // appends in a launch of its own first
   const int kvt = pool->desc.kv_type;
   const bool fold = k_new && plan_folds_append(pool, a, pl);
   const bool rope_fold = fold && rope.style != ROPE_NONE && plan_folds_rope(pool, a, pl);
