@@ -21,7 +21,8 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
   d.kv_type = kv;
   int waves = 0;
   int64_t part = 0;
-  if (!small_plan(&a, d, resident, (int64_t)kBS * dim * kv_esz(kv), &waves, &part)) return;
+  const WgResident waves_at = {resident / 4, resident / 2, resident, resident};  // as with much LDS
+  if (!small_plan(&a, d, waves_at, (int64_t)kBS * dim * kv_esz(kv), &waves, &part)) return;
   const int64_t nb = (longest + kBS - 1) / kBS;
   const bool range = waves >= 1 && waves <= kWgMaxWaves && part >= 1 && part <= nb;
   // a wave holds the ids of 256 blocks, whatever the lengths turn out to be
@@ -31,9 +32,10 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
            (long long)longest, (long long)sum, kv, dim, (long long)resident, waves, (long long)part);
 }
 
-// One sequence of `longest` tokens and n - 1 of `rest`, 2,048 resident waves: whether the rule
-// takes the batch (measured both ways: us of the small plan, of stream-K).
-struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; };
+// One sequence of `longest` tokens and n - 1 of `rest`, 2,048 resident waves (one_wave of them in
+// workgroups of one): whether the rule takes the batch (measured both ways: us of the small plan,
+// of stream-K or, for equal lengths, of the plan for uniform batches; 0: not measured).
+struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; int one_wave = 2048; };
 static const Skewed kSkewed[] = {
     {VK_KV_I8_BLK, 8, 64, 500, 200, true, 12.3, 18.9},   {VK_KV_I8_BLK, 8, 64, 16000, 200, false, 122.3, 33.6},
     {VK_KV_I8_BLK, 8, 128, 4000, 100, false, 67.2, 23.4}, {VK_KV_I8_BLK, 8, 16, 8000, 500, true, 17.1, 29.6},
@@ -43,7 +45,9 @@ static const Skewed kSkewed[] = {
     {VK_KV_I8_REF, 8, 40, 8000, 200, false, 67.7, 30.4}, {VK_KV_I8_REF, 8, 24, 8000, 300, true, 24.8, 31.1},
     {VK_KV_F32, 8, 24, 16000, 300, false, 84.4, 65.2},   {VK_KV_F32, 8, 16, 16000, 500, true, 54.9, 65.3},
     {VK_KV_F32, 8, 200, 2000, 60, false, 211.2, 50.0},   {VK_KV_F32, 8, 24, 500, 300, true, 24.4, 32.3},
-    {VK_KV_F16, 4, 199, 335, 180, true, 12.8, 16.9},
+    {VK_KV_F16, 4, 199, 335, 180, true, 12.8, 16.9},     {VK_KV_I8_BLK, 8, 182, 160, 145, false, 36.9, 26.7, 512},
+    {VK_KV_I8_BLK, 8, 182, 160, 145, true, 0, 0},         {VK_KV_I8_BLK, 8, 157, 79, 79, false, 24.0, 18.7, 512},
+    {VK_KV_I8_REF, 8, 141, 68, 68, false, 31.5, 24.5, 1024}, {VK_KV_I8_REF, 8, 141, 68, 68, true, 0, 0},
 };
 
 static void check_skewed(const Skewed& c) {
@@ -58,9 +62,10 @@ static void check_skewed(const Skewed& c) {
   d.kv_type = c.kv;
   int waves = 0;
   int64_t part = 0;
-  if (small_plan(&a, d, 2048, (int64_t)kBS * 128 * kv_esz(c.kv), &waves, &part) == c.small) return;
+  const WgResident waves_at = {c.one_wave, 2048, 2048, 2048};
+  if (small_plan(&a, d, waves_at, (int64_t)kBS * 128 * kv_esz(c.kv), &waves, &part) == c.small) return;
   if (bad++ < 10)
-    printf("skewed: kv %d, %d x %d heads, longest %d, rest %d: small %d (%.1f us, stream-K %.1f)\n", c.kv, c.n, c.hkv,
+    printf("skewed: kv %d, %d x %d heads, longest %d, rest %d: small %d (%.1f us, else %.1f)\n", c.kv, c.n, c.hkv,
            c.longest, c.rest, !c.small, c.us, c.sk_us);
 }
 

@@ -124,8 +124,9 @@ struct vk_ctx {
   int decode_kind = VK_DECODE_AUTO;
   int decode_sched = VK_SCHED_AUTO;
   int n_cu = 256;
-  std::mutex res_mu;                                   // guards resident
+  std::mutex res_mu;                                   // guards resident, wg_resident
   std::unordered_map<std::string, int64_t> resident;  // kernel -> resident waves
+  std::unordered_map<std::string, WgResident> wg_resident;
 
   hipFunction_t fn(const std::string& name) const {
     auto it = fns.find(name);
@@ -250,6 +251,19 @@ int64_t resident_waves(vk_ctx* ctx, const std::string& name, int block = 64) {
   return waves;
 }
 
+// The same of a workgroup-split kernel in workgroups of 1, 2, 4 and 8 waves.
+WgResident wg_resident_waves(vk_ctx* ctx, const std::string& name) {
+  {
+    std::lock_guard<std::mutex> lk(ctx->res_mu);
+    auto it = ctx->wg_resident.find(name);
+    if (it != ctx->wg_resident.end()) return it->second;
+  }
+  WgResident r;
+  for (size_t i = 0; i < r.size(); ++i) r[i] = resident_waves(ctx, name, 64 << i);
+  std::lock_guard<std::mutex> lk(ctx->res_mu);
+  ctx->wg_resident[name] = r;
+  return r;
+}
 
 int check_pool(const vk_ctx* ctx, const vk_pool* pool) {
   if (!ctx) return fail(VK_ERR_NOT_WIRED, "context is null");
@@ -844,9 +858,10 @@ int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, Decod
   int64_t part = 0;
   int waves = 0;
   const std::string wg = decode_wg_name(d.kv_type, G, a->q_dtype, d64);
-  const int64_t wg_waves = ctx ? resident_waves(ctx, wg, 64 * kWgMaxWaves) : 2048;
+  const WgResident wg_res = ctx ? wg_resident_waves(ctx, wg) : WgResident{2048, 2048, 2048, 2048};
+  const int64_t wg_waves = wg_res[3];
   if (sched == VK_SCHED_AUTO && !valu && P == 0 && G <= kMaxGroupTile &&
-      small_plan(a, d, wg_waves, pool->geom.tile_bytes, &waves, &part)) {
+      small_plan(a, d, wg_res, pool->geom.tile_bytes, &waves, &part)) {
     const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
     pl->stream_k = false;
     pl->wg_waves = waves;

@@ -4,6 +4,7 @@
 #include "velokv.h"
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 
 namespace velokv {
@@ -59,6 +60,9 @@ constexpr int64_t kWaveRate8 = 5400, kWaveRate = 9000;
 constexpr int64_t kMergeNs = 3400;
 constexpr int64_t kSkFixedNs = 9000, kSkPartialNs = 80;
 
+// Waves of a workgroup-split kernel on the device at once in workgroups of 1, 2, 4, 8.
+using WgResident = std::array<int64_t, 4>;
+
 inline bool uniform_batch(const vk_decode_args* a) {
   return a->sum_context_len > 0 &&
          (double)a->sum_context_len >= 0.97 * (double)a->n_seqs * (double)a->max_context_len;
@@ -66,13 +70,14 @@ inline bool uniform_batch(const vk_decode_args* a) {
 
 // Workgroup split of a small batch (VK_SCHED_AUTO): *waves waves per (sequence,
 // partition of *part_blocks blocks, KV head); false when the batch is too large
-// for it, or a wave's share of its longest context is. waves_total: resident waves
-// of the kernel; tile: K bytes of one block and KV head. The lengths' sum only steers the choice: any lengths up to
+// for it, or a wave's share of its longest context is. tile: K bytes of one
+// block and KV head. The lengths' sum only steers the choice: any lengths up to
 // max_context_len are computed whatever it says.
-inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves_total, int64_t tile, int* waves,
+inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, const WgResident& resident, int64_t tile, int* waves,
                        int64_t* part_blocks) {
   const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
   const int64_t pairs = (int64_t)a->n_seqs * d.n_kv_heads;
+  const int64_t waves_total = resident[3];  // of kWgMaxWaves
   if (pairs <= 0 || nb <= 0 || pairs > waves_total) return false;
   // lengths the host does not know (any up to max_context_len) stay with stream-K,
   // which balances whatever they are
@@ -87,8 +92,14 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t w
   // split-K, whose result needs no combining (5.6 us per call at two int8 blocks;
   // fp16 split-K runs the vector kernel, 13.0 us at 16 x 32 tokens against 5.6)
   if (uniform_batch(a) && d.kv_type != VK_KV_F16 && nb * kv_esz(d.kv_type) <= 4) return false;
-  int nw = nb <= kWgMaxWaves ? kWgMaxWaves / 2 : kWgMaxWaves;
-  while (nw > 1 && pairs * nw > waves_total) nw /= 2;
+  int nw = nb <= kWgMaxWaves ? kWgMaxWaves / 2 : kWgMaxWaves, lg = nb <= kWgMaxWaves ? 2 : 3;
+  while (nw > 1 && pairs * nw > waves_total) nw /= 2, --lg;
+  // each workgroup takes the LDS of kWgMaxWaves waves whatever it has (64 KB with 7
+  // query heads per KV head or 64-dim tiles, two on a CU), so those of few waves may
+  // take turns: 116 x 8 heads of 105 fp16 tokens, 7 query heads per KV head, 24.9 us,
+  // split-K 16.0
+  const int64_t turns = (pairs * nw + resident[lg] - 1) / resident[lg];
+  if (turns > 1 && uniform_batch(a)) return false;
   *waves = nw;
   *part_blocks = nb;
   if (nw == kWgMaxWaves) {
@@ -104,7 +115,7 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, int64_t w
   if (!uniform_batch(a) && a->n_seqs > 1) {
     const int64_t even = sum * d.n_kv_heads * 2 * tile / waves_total;  // bytes of a wave if all had the same
     const int64_t wave = (*part_blocks + nw - 1) / nw * 2 * tile;
-    const int64_t late = std::max<int64_t>(0, wave - even) * 1000 / (nw == kWgMaxWaves ? kWaveRate8 : kWaveRate) +
+    const int64_t late = std::max<int64_t>(0, turns * wave - even) * 1000 / (nw == kWgMaxWaves ? kWaveRate8 : kWaveRate) +
                          (*part_blocks < nb ? kMergeNs : 0);
     const int64_t share = std::max<int64_t>(1, (sum * d.n_kv_heads + kSkPenalty * pairs) / waves_total);
     if (late > kSkFixedNs + kSkPartialNs * (nb / share)) return false;
