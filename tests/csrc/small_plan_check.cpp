@@ -17,7 +17,10 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
   a.n_seqs = n_seqs;
   a.max_context_len = (int32_t)longest;
   a.sum_context_len = sum;
+  a.n_heads = hkv * 4;
+  a.q_dtype = VK_DT_F16;
   d.n_kv_heads = hkv;
+  d.head_dim = dim;
   d.kv_type = kv;
   int waves = 0;
   int64_t part = 0;
@@ -35,7 +38,7 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
 // One sequence of `longest` tokens and n - 1 of `rest`, 2,048 resident waves (one_wave of them in
 // workgroups of one): whether the rule takes the batch (measured both ways: us of the small plan,
 // of stream-K or, for equal lengths, of the plan for uniform batches; 0: not measured).
-struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; int one_wave = 2048; };
+struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; int one_wave = 2048, G = 4; };
 static const Skewed kSkewed[] = {
     {VK_KV_I8_BLK, 8, 64, 500, 200, true, 12.3, 18.9},   {VK_KV_I8_BLK, 8, 64, 16000, 200, false, 122.3, 33.6},
     {VK_KV_I8_BLK, 8, 128, 4000, 100, false, 67.2, 23.4}, {VK_KV_I8_BLK, 8, 16, 8000, 500, true, 17.1, 29.6},
@@ -48,6 +51,15 @@ static const Skewed kSkewed[] = {
     {VK_KV_F16, 4, 199, 335, 180, true, 12.8, 16.9},     {VK_KV_I8_BLK, 8, 182, 160, 145, false, 36.9, 26.7, 512},
     {VK_KV_I8_BLK, 8, 182, 160, 145, true, 0, 0},         {VK_KV_I8_BLK, 8, 157, 79, 79, false, 24.0, 18.7, 512},
     {VK_KV_I8_REF, 8, 141, 68, 68, false, 31.5, 24.5, 1024}, {VK_KV_I8_REF, 8, 141, 68, 68, true, 0, 0},
+    // uniform fp16: seven, one and four query heads per KV head
+    {VK_KV_F16, 8, 35, 37, 37, false, 11.2, 9.5, 2048, 7},   {VK_KV_F16, 8, 4, 41, 41, false, 9.9, 9.1, 2048, 7},
+    {VK_KV_F16, 8, 23, 107, 107, true, 10.8, 11.1, 2048, 7}, {VK_KV_F16, 8, 20, 4861, 4861, false, 78.3, 70.7, 2048, 7},
+    {VK_KV_F16, 8, 1, 18, 18, true, 7.3, 7.9, 2048, 7},      {VK_KV_F16, 8, 34, 1469, 1469, false, 52.1, 39.2, 2048, 1},
+    {VK_KV_F16, 8, 54, 23, 23, false, 9.0, 7.4, 2048, 1},    {VK_KV_F16, 8, 6, 152, 152, true, 9.6, 9.5, 2048, 1},
+    {VK_KV_F16, 8, 3, 288, 288, true, 11.0, 14.1, 2048, 1},  {VK_KV_F16, 8, 40, 128, 128, true, 11.7, 25.5, 2048, 4},
+    {VK_KV_F16, 8, 18, 6985, 6985, false, 107.1, 91.5, 2048, 4}, {VK_KV_F16, 8, 29, 2070, 2070, true, 42.1, 58.3, 2048, 4},
+    // and of other types, a few long contexts and many short ones
+    {VK_KV_F32, 8, 6, 243, 243, true, 17.8, 33.5},           {VK_KV_I8_BLK, 8, 3, 771, 771, true, 18.5, 21.1},
 };
 
 static void check_skewed(const Skewed& c) {
@@ -58,7 +70,10 @@ static void check_skewed(const Skewed& c) {
   a.n_seqs = c.n;
   a.max_context_len = c.longest;
   a.sum_context_len = c.longest + (int64_t)(c.n - 1) * c.rest;
+  a.n_heads = c.G * c.hkv;
+  a.q_dtype = VK_DT_F16;
   d.n_kv_heads = c.hkv;
+  d.head_dim = 128;
   d.kv_type = c.kv;
   int waves = 0;
   int64_t part = 0;

@@ -60,6 +60,15 @@ constexpr int64_t kWaveRate8 = 5400, kWaveRate = 9000;
 constexpr int64_t kMergeNs = 3400;
 constexpr int64_t kSkFixedNs = 9000, kSkPartialNs = 80;
 
+// A uniform batch keeps the plan for uniform batches when its longest wave, of at
+// least kLongWave bytes, streams past the even share for longer than that plan's
+// merge of more and shorter pieces takes (the workgroups of 144 x 8-wave calls leave
+// 112 of 256 CUs empty): 5 us, 18 us where it is the vector kernel with 4 or 8 query
+// heads per KV head. 160 pairs of 4,861 fp16 tokens, 7 query heads per KV head, 78.3 us
+// against 70.7; 170 of 1,114 24.6 against 25.8.
+constexpr int64_t kLongWave = 60000;
+constexpr int64_t kSplitNs = 5000, kVectorNs = 18000;
+
 // Waves of a workgroup-split kernel on the device at once in workgroups of 1, 2, 4, 8.
 using WgResident = std::array<int64_t, 4>;
 
@@ -92,6 +101,22 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, const WgR
   // split-K, whose result needs no combining (5.6 us per call at two int8 blocks;
   // fp16 split-K runs the vector kernel, 13.0 us at 16 x 32 tokens against 5.6)
   if (uniform_batch(a) && d.kv_type != VK_KV_F16 && nb * kv_esz(d.kv_type) <= 4) return false;
+  // uniform fp16 ones where the plan for uniform batches is not the vector kernel with 4
+  // or 8 query heads per KV head (slow: 40 x 128 tokens 25.5 us against 11.7): one wave
+  // per context needs no combining up to six blocks (47 x 8 heads of 48 tokens 10.2 us
+  // against 12.4), with up to two query heads per KV head where it fills the SIMDs (41 x 8
+  // heads of 23-207 tokens 7.4-12.3 against 9.0-13.1), and over 128-dim tiles past one
+  // workgroup of eight waves a CU at any length (34 x 8 heads of 1,469 39.2 against 52.1).
+  // One sequence has the append folded in instead (18 tokens 7.1 us against 8.5).
+  const int G = a->n_heads / d.n_kv_heads;
+  const bool vec = d.kv_type == VK_KV_F16 && a->q_dtype == VK_DT_F16 && d.head_dim == 128 &&
+                   (G == 1 || G == 2 || G == 4 || G == 8);
+  const bool slow = vec && G >= 4;
+  if (uniform_batch(a) && d.kv_type == VK_KV_F16 && !slow) {
+    const bool over = pairs * kWgMaxWaves > waves_total, wide = tile >= kBS * 128 * 2;
+    if (wide && over) return false;
+    if (!over && a->n_seqs > 1 && nb <= 6 && (!vec || pairs > 128)) return false;
+  }
   int nw = nb <= kWgMaxWaves ? kWgMaxWaves / 2 : kWgMaxWaves, lg = nb <= kWgMaxWaves ? 2 : 3;
   while (nw > 1 && pairs * nw > waves_total) nw /= 2, --lg;
   // each workgroup takes the LDS of kWgMaxWaves waves whatever it has (64 KB with 7
@@ -112,11 +137,14 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, const WgR
     part = std::max(part, std::max<int64_t>(8, kMinPartBytes / (2 * tile)));
     if ((nb - part) * 2 * tile > kMergeBytes && (nb + part - 1) / part * pairs <= kMaxPartWgs) *part_blocks = part;
   }
-  if (!uniform_batch(a) && a->n_seqs > 1) {
-    const int64_t even = sum * d.n_kv_heads * 2 * tile / waves_total;  // bytes of a wave if all had the same
-    const int64_t wave = (*part_blocks + nw - 1) / nw * 2 * tile;
-    const int64_t late = std::max<int64_t>(0, turns * wave - even) * 1000 / (nw == kWgMaxWaves ? kWaveRate8 : kWaveRate) +
-                         (*part_blocks < nb ? kMergeNs : 0);
+  // bytes of the longest wave, of a wave if all had the same, and the time between them
+  const int64_t even = sum * d.n_kv_heads * 2 * tile / waves_total;
+  const int64_t wave = (*part_blocks + nw - 1) / nw * 2 * tile;
+  int64_t late = std::max<int64_t>(0, turns * wave - even) * 1000 / (nw == kWgMaxWaves ? kWaveRate8 : kWaveRate);
+  if (uniform_batch(a)) {
+    if (wave >= kLongWave && late > (slow ? kVectorNs : kSplitNs)) return false;
+  } else if (a->n_seqs > 1) {
+    if (*part_blocks < nb) late += kMergeNs;
     const int64_t share = std::max<int64_t>(1, (sum * d.n_kv_heads + kSkPenalty * pairs) / waves_total);
     if (late > kSkFixedNs + kSkPartialNs * (nb / share)) return false;
   }
