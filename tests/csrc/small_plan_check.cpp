@@ -38,7 +38,7 @@ static void check(int n_seqs, int hkv, int64_t longest, int64_t sum, int kv, int
 // One sequence of `longest` tokens and n - 1 of `rest`, 2,048 resident waves (one_wave of them in
 // workgroups of one): whether the rule takes the batch (measured both ways: us of the small plan,
 // of stream-K or, for equal lengths, of the plan for uniform batches; 0: not measured).
-struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; int one_wave = 2048, G = 4; };
+struct Skewed { int kv, hkv, n, longest, rest; bool small; double us, sk_us; int one_wave = 2048, G = 4, dim = 128; };
 static const Skewed kSkewed[] = {
     {VK_KV_I8_BLK, 8, 64, 500, 200, true, 12.3, 18.9},   {VK_KV_I8_BLK, 8, 64, 16000, 200, false, 122.3, 33.6},
     {VK_KV_I8_BLK, 8, 128, 4000, 100, false, 67.2, 23.4}, {VK_KV_I8_BLK, 8, 16, 8000, 500, true, 17.1, 29.6},
@@ -51,6 +51,7 @@ static const Skewed kSkewed[] = {
     {VK_KV_F16, 4, 199, 335, 180, true, 12.8, 16.9},     {VK_KV_I8_BLK, 8, 182, 160, 145, false, 36.9, 26.7, 512},
     {VK_KV_I8_BLK, 8, 182, 160, 145, true, 0, 0},         {VK_KV_I8_BLK, 8, 157, 79, 79, false, 24.0, 18.7, 512},
     {VK_KV_I8_REF, 8, 141, 68, 68, false, 31.5, 24.5, 1024}, {VK_KV_I8_REF, 8, 141, 68, 68, true, 0, 0},
+    {VK_KV_I8_BLK, 8, 182, 160, 145, false, 37.1, 26.7, 512, 7, 64},
     // uniform fp16: seven, one and four query heads per KV head
     {VK_KV_F16, 8, 35, 37, 37, false, 11.2, 9.5, 2048, 7},   {VK_KV_F16, 8, 4, 41, 41, false, 9.9, 9.1, 2048, 7},
     {VK_KV_F16, 8, 23, 107, 107, true, 10.8, 11.1, 2048, 7}, {VK_KV_F16, 8, 20, 4861, 4861, false, 78.3, 70.7, 2048, 7},
@@ -73,12 +74,12 @@ static void check_skewed(const Skewed& c) {
   a.n_heads = c.G * c.hkv;
   a.q_dtype = VK_DT_F16;
   d.n_kv_heads = c.hkv;
-  d.head_dim = 128;
+  d.head_dim = c.dim;
   d.kv_type = c.kv;
   int waves = 0;
   int64_t part = 0;
   const WgResident waves_at = {c.one_wave, 2048, 2048, 2048};
-  if (small_plan(&a, d, waves_at, (int64_t)kBS * 128 * kv_esz(c.kv), &waves, &part) == c.small) return;
+  if (small_plan(&a, d, waves_at, (int64_t)kBS * c.dim * kv_esz(c.kv), &waves, &part) == c.small) return;
   if (bad++ < 10)
     printf("skewed: kv %d, %d x %d heads, longest %d, rest %d: small %d (%.1f us, else %.1f)\n", c.kv, c.n, c.hkv,
            c.longest, c.rest, !c.small, c.us, c.sk_us);

@@ -58,6 +58,7 @@ constexpr int64_t kMaxPartWgs = 2048;
 // against 19.8, one of 1,000 22.4 against 20.2.
 constexpr int64_t kWaveRate8 = 5400, kWaveRate = 9000;
 constexpr int64_t kMergeNs = 3400;
+constexpr int64_t kTurnNs = 6000;  // each further turn of workgroups on a CU
 constexpr int64_t kSkFixedNs = 9000, kSkPartialNs = 80;
 
 // A uniform batch keeps the plan for uniform batches when its longest wave, of at
@@ -144,7 +145,7 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, const WgR
   if (uniform_batch(a)) {
     if (wave >= kLongWave && late > (slow ? kVectorNs : kSplitNs)) return false;
   } else if (a->n_seqs > 1) {
-    if (*part_blocks < nb) late += kMergeNs;
+    late += (turns - 1) * kTurnNs + (*part_blocks < nb ? kMergeNs : 0);
     const int64_t share = std::max<int64_t>(1, (sum * d.n_kv_heads + kSkPenalty * pairs) / waves_total);
     if (late > kSkFixedNs + kSkPartialNs * (nb / share)) return false;
   }
