@@ -29,6 +29,7 @@ def patterns():
         "drafts": b(7, 5, 13) + b(4, 12, 16) + b(6, 0, 4) + b(8, 15, 16),     # 8-token drafts, one over two blocks
         "single": [7 * BS + 5, 4 * BS, 9 * BS + 15, 10 * BS + 2],
         "padding": [-1, 7 * BS + 5, -1, 7 * BS + 6, 2 * BS, -1, -1, 2 * BS + 1, 5 * BS, N_BLOCKS * BS, -1],
+        "wrap": b(2, 8, 16) + b(2, 0, 8) + b(4, 14, 16) + [4 * BS + 13],        # goes on in a block filled to its end
         "order": [2 * BS + 1, 2 * BS, 2 * BS + 3, 2 * BS + 2, 6 * BS + 1, 6 * BS + 2, 6 * BS + 4],
     }
 

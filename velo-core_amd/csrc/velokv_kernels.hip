@@ -3390,16 +3390,16 @@ DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint
     unsigned long long old = 0;
     if (claim) old = __hip_atomic_exchange(&P.claim[slot / BS], me, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // tokens in consecutive slots of the block, and nothing of the block after them
-    // (the block's end, the call's end or a token of another block; no padding or
-    // reordering within): all at once (a half-split rotation needs its partners in
-    // the lanes that path gives them; one token is done sooner with its dims over
-    // the wave, 5.4 us a call against 7.4)
+    // (the call's end or a token of another block; no padding or reordering within,
+    // and no token that goes on in a block filled to its end): all at once (a half-split
+    // rotation needs its partners in the lanes that path gives them; one token is done
+    // sooner with its dims over the wave, 5.4 us a call against 7.4)
     const int o0 = (int)(slot % BS);
     const uint64_t same = __builtin_amdgcn_ballot_w64(lane >= j && ms64 == slot + (lane - j)) >> j;
     const int m = min(BS - o0, __builtin_ctzll(~same));
     const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m < 64
     const int nx = __shfl((int)(ms64 / BS), after != 0 ? j + m + __builtin_ctzll(after) : 0, WAVE);
-    if (m > 1 && (o0 + m == BS || (after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok)) &&
+    if (m > 1 && (after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok) &&
         (IS_V || P.rope != ROPE_HALF || P.g.io_hd == D))
       append_blk_tile<IS_V, D>(P, src, codes, scales, w0 + j, m, o0, slot / BS, h);
     else
