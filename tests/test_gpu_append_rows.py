@@ -31,6 +31,7 @@ def patterns():
         "padding": [-1, 7 * BS + 5, -1, 7 * BS + 6, 2 * BS, -1, -1, 2 * BS + 1, 5 * BS, N_BLOCKS * BS, -1],
         "wrap": b(2, 8, 16) + b(2, 0, 8) + b(4, 14, 16) + [4 * BS + 13],        # goes on in a block filled to its end
         "order": [2 * BS + 1, 2 * BS, 2 * BS + 3, 2 * BS + 2, 6 * BS + 1, 6 * BS + 2, 6 * BS + 4],
+        "contiguous": b(8, 0, 16) + b(9, 0, 16) + b(10, 0, 16) + b(11, 0, 16),  # 64 slots in a row from the call's start
     }
 
 

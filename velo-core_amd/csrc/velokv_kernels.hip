@@ -3396,8 +3396,8 @@ DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint
     // sooner with its dims over the wave, 5.4 us a call against 7.4)
     const int o0 = (int)(slot % BS);
     const uint64_t same = __builtin_amdgcn_ballot_w64(lane >= j && ms64 == slot + (lane - j)) >> j;
-    const int m = min(BS - o0, __builtin_ctzll(~same));
-    const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m < 64
+    const int m = __builtin_ctzll(~same | (1ull << (BS - o0)));
+    const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m <= BS
     const int nx = __shfl((int)(ms64 / BS), after != 0 ? j + m + __builtin_ctzll(after) : 0, WAVE);
     if (m > 1 && (after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok) &&
         (IS_V || P.rope != ROPE_HALF || P.g.io_hd == D))
