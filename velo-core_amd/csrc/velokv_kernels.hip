@@ -999,12 +999,18 @@ DEV float div_scale(float x, float s, float y) {
   const float q = x * y;
   return fmaf(fmaf(-q, s, x), y, q);
 }
+DEV float blk_clamp(float q) { return fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f); }
 DEV float blk_rne(float x, float s, float y) {
   const float q = s < __builtin_huge_valf() ? div_scale(x, s, y) : x / s;  // (wave-uniform)
-  return fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f);
+  return blk_clamp(q);
 }
 DEV int blk_requant(int c, float s_old, float s_new, float y) { return (int)blk_rne((float)c * s_old, s_new, y); }
 DEV int blk_code(float x, float s_new, float y) { return s_new > 0.f ? (int)blk_rne(x, s_new, y) : 0; }
+// The same by a division of each value, for the append folded into a decode: beside a
+// piece's stages the inverse and the scale test spilled up to five registers more
+// (stream-K with RoPE, 2 to 16 query heads per KV head).
+DEV int blk_requant(int c, float s_old, float s_new) { return (int)blk_clamp((float)c * s_old / s_new); }
+DEV int blk_code(float x, float s_new) { return s_new > 0.f ? (int)blk_clamp(x / s_new) : 0; }
 
 // The rule over a block whose codes are in registers (cd) and whose scale is
 // s_old (bits s_bits).
@@ -1116,15 +1122,15 @@ DEV int byte_at(uint32_t w, int k) { return (int)(int8_t)(uint8_t)(w >> (8 * k))
 // 64-dim row read the codes 64 dims below and store nothing. K codes of token u
 // at dims 2 lane, 2 lane + 1 are two adjacent bytes; V codes of the token pair
 // 2p, 2p + 1 are four (dim 2 lane: tokens 2p, 2p + 1; then dim 2 lane + 1).
-DEV uint32_t blk_requant4(uint32_t w, float s_old, float s_new, float y) {
+DEV uint32_t blk_requant4(uint32_t w, float s_old, float s_new) {
   uint32_t r = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) r |= (uint32_t)(blk_requant(byte_at(w, k), s_old, s_new, y) & 0xFF) << (8 * k);
+  for (int k = 0; k < 4; ++k) r |= (uint32_t)(blk_requant(byte_at(w, k), s_old, s_new) & 0xFF) << (8 * k);
   return r;
 }
-DEV uint4 blk_requant16(uint4 v, float s_old, float s_new, float y) {
-  return make_uint4(blk_requant4(v.x, s_old, s_new, y), blk_requant4(v.y, s_old, s_new, y),
-                    blk_requant4(v.z, s_old, s_new, y), blk_requant4(v.w, s_old, s_new, y));
+DEV uint4 blk_requant16(uint4 v, float s_old, float s_new) {
+  return make_uint4(blk_requant4(v.x, s_old, s_new), blk_requant4(v.y, s_old, s_new), blk_requant4(v.z, s_old, s_new),
+                    blk_requant4(v.w, s_old, s_new));
 }
 
 template <bool IS_V, int D>
@@ -1140,15 +1146,14 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
   const float s_new = blk_scale(s_old, s_bits, f.x[e][0], f.x[e][1]);
   const bool grew = s_new > s_old && o > 0;  // requantize the tokens before o
   uint8_t* tile = const_cast<uint8_t*>(IS_V ? P.vc : P.kc) + f.tix * P.tile_bytes;
-  const float y = blk_inv(s_new);
-  const int c0 = blk_code(f.x[e][0], s_new, y), c1 = blk_code(f.x[e][1], s_new, y);
+  const int c0 = blk_code(f.x[e][0], s_new), c1 = blk_code(f.x[e][1], s_new);
   if constexpr (!IS_V) {
     if (grew) {
 #pragma unroll
       for (int j = 0; j < D / 64; ++j) {
         const int q = lane + 64 * j;
         if ((q % (D / 2)) / (D / 32) < o)  // the piece's token
-          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.kq[j], s_old, s_new, y);
+          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.kq[j], s_old, s_new);
       }
     }
     if (st)
@@ -1159,7 +1164,7 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
       for (int j = 0; j < D / 64; ++j) {
         const int q = lane + 64 * j;
         if (q / (D / 8) < (o >> 1))  // the piece's token pair
-          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.vq[j], s_old, s_new, y);
+          reinterpret_cast<uint4*>(tile)[q] = blk_requant16(f.vq[j], s_old, s_new);
       }
     }
     if (st) {  // bytes: (2P, d0), (2P + 1, d0), (2P, d0 + 1), (2P + 1, d0 + 1)
@@ -1167,8 +1172,8 @@ DEV uint32_t fold_finish_one(FoldIn& f, const DecodeParams& P) {
       if (o & 1) {  // token o - 1 (requantized when the scale grew), then token o
         int a0 = byte_at(w, 0), a1 = byte_at(w, 2);
         if (grew) {
-          a0 = blk_requant(a0, s_old, s_new, y);
-          a1 = blk_requant(a1, s_old, s_new, y);
+          a0 = blk_requant(a0, s_old, s_new);
+          a1 = blk_requant(a1, s_old, s_new);
         }
         w = (uint32_t)(a0 & 0xFF) | ((uint32_t)(c0 & 0xFF) << 8) | ((uint32_t)(a1 & 0xFF) << 16) |
             ((uint32_t)(c1 & 0xFF) << 24);
