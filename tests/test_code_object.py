@@ -37,3 +37,8 @@ def test_stream_k_fold_spills(kernels):
     assert len(got) == 24
     for n, (_, spills) in got.items():
         assert spills <= STREAM_K_SPILLS.get(n.removeprefix("vk_decode_sk_kv3_"), 0), n
+
+
+@pytest.mark.parametrize("name", ["vk_decode_merge", "vk_decode_merge_sk"])
+def test_merges_use_no_scratch_memory(kernels, name):
+    assert kernels[name] == (0, 0)

@@ -2827,9 +2827,14 @@ DEV void merge_row(const MergeParams& P, int64_t out_row, int np, PR pr, float2 
   for (int p0 = 0; p0 < np; p0 += WAVE) {
     float w = 0.f;
     if (p0 + lane < np) {
-      const float2 m = p0 == 0 ? m0 : ml[pr(p0 + lane)];
-      w = (m.x == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m.x - M);
-      L = fmaf(w, m.y, L);
+      float mx = m0.x, my = m0.y;
+      if (p0 > 0) {  // (no select between m0 and the load: it became one of addresses, with m0 in scratch memory)
+        const float2 m = ml[pr(p0 + lane)];
+        mx = m.x;
+        my = m.y;
+      }
+      w = (mx == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(mx - M);
+      L = fmaf(w, my, L);
     }
     const int cnt = min(WAVE, np - p0);
     for (int k0 = 0; k0 < cnt; k0 += 8) {
