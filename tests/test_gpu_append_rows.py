@@ -123,3 +123,21 @@ def test_append_prompt_of_many_windows(ctx, kv):
     ctx.sync()
     O.append(ref, k, v, sl)
     assert_layer_equal(pool, 0, ref)
+
+
+def test_append_nan_scale(ctx):
+    """A per-token int8 row of 128 NaN has the scale NaN, and of fewer dims (the tile's others are zeros)
+    0, in a short call (a workgroup per token) as in a long one (rows); its codes are 0 (parity unpinned)."""
+    for hd, want in ((128, np.nan), (96, 0.0), (64, 0.0)):
+        for lead in (0, 1101):
+            print(f"append NaN rows hd={hd} lead={lead}", flush=True)
+            pool = velokv.Pool(ctx, 1, 2, BS, HKV, hd, O.I8_REF)
+            k = np.full((lead + 1, HKV, hd), np.nan, np.float32)
+            ctx.append(pool, 0, ctx.upload(k), ctx.upload(k), velokv.DT_F32, ctx.upload(np.array([-1] * lead + [BS], np.int64)),
+                       lead + 1)
+            ctx.sync()
+            got = pool.download_layer(0)
+            for key in ("ks", "vs"):
+                scale = got[key].view(np.float32).reshape(2, HKV, BS)[1, :, 0]
+                assert np.array_equal(scale, np.full(HKV, want, np.float32), equal_nan=True), (key, scale)
+            assert not got["k"].any() and not got["v"].any()

@@ -3502,9 +3502,9 @@ DEV float max16(float m) {  // over the row's sixteen lanes
 template <int KV>
 DEV void row_codes(const Row8& r, uint32_t (&w)[8], float& scale) {
   if constexpr (KV == KV_I8_REF) {
-    float m = 0.f;
+    float m = fabsf(r.x[0]);  // (a row of 128 NaN has the scale NaN, as append_token gives it)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(r.x[k]));
+    for (int k = 1; k < 8; ++k) m = fmaxf(m, fabsf(r.x[k]));
     m = max16(m);
     scale = m / 127.0f;
     const float inv = m > 0.f ? 127.0f / m : 0.f;
