@@ -141,3 +141,34 @@ def test_append_nan_scale(ctx):
                 scale = got[key].view(np.float32).reshape(2, HKV, BS)[1, :, 0]
                 assert np.array_equal(scale, np.full(HKV, want, np.float32), equal_nan=True), (key, scale)
             assert not got["k"].any() and not got["v"].any()
+
+
+def test_append_f16_bits(ctx):
+    """fp16 rows go into an fp16 pool of 128 dims bit for bit, signalling NaN included, V pairs and single
+    tokens, in a short call as in a long one; unrotated K rows do, and V rows whatever K does."""
+    r = np.random.default_rng(4300)
+    n, N = 3, 3 * HKV * 128
+    where = np.arange(1, N + 1).reshape(n, HKV, 128).astype(np.float16)  # (integers: exact in fp16)
+    slots = np.array([BS + 4, BS + 5, 7], np.int64)
+    at = O.Layer(2, HKV, BS, 128, O.F16)
+    O.append(at, where, where, slots)
+    bits = r.integers(0, 1 << 16, N + 1).astype(np.uint16)
+    bits[1:40] = np.arange(0x7C01, 0x7C01 + 39)  # signalling NaN
+    bits[0] = 0
+    rows16 = bits[where.astype(np.int64)]
+    for lead in (0, 1101):
+        for rope in (False, True):
+            print(f"append fp16 bits lead={lead} rope={rope}", flush=True)
+            pool = velokv.Pool(ctx, 1, 2, BS, HKV, 128, O.F16)
+            x = ctx.upload(np.concatenate([np.zeros((lead, HKV, 128), np.uint16), rows16]))
+            sl = ctx.upload(np.concatenate([np.full(lead, -1, np.int64), slots]))
+            if rope:
+                ctx.append_rope(pool, 0, x, x, velokv.DT_F16, ctx.upload(np.zeros(lead + n, np.int32)), sl, lead + n,
+                                ctx.upload(velokv.rope_table(4, 128, 10000.0)), 4, O.ROPE_HALF)
+            else:
+                ctx.append(pool, 0, x, x, velokv.DT_F16, sl, lead + n)
+            ctx.sync()
+            got = pool.download_layer(0)
+            for key in ("v",) if rope else ("k", "v"):
+                ref = bits[np.frombuffer(getattr(at, key).tobytes(), np.float16).astype(np.int64)]
+                assert np.array_equal(got[key].view(np.uint16), ref), key

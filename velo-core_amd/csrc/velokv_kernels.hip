@@ -3434,8 +3434,9 @@ struct Row8 { float x[8]; };  // dims a .. a + 3, b .. b + 3
 
 // N rows of io elements (element offsets `row`) of src at the lane's dims. All
 // loads of the rows go out in one branch on the type: the compiler waits for a
-// branch's loads at its end, so a branch per row was a round trip per row.
-template <int N>
+// branch's loads at its end, so a branch per row was a round trip per row. BITS: fp16
+// values as their bits.
+template <int N, bool BITS>
 DEV void load_rows8(const void* src, int dtype, const int64_t (&row)[N], int a, int b, bool in, Row8 (&r)[N]) {
   const int oa = in ? a : 0, ob = in ? b : 0;
   if (dtype == DT_F16) {
@@ -3450,8 +3451,9 @@ DEV void load_rows8(const void* src, int dtype, const int64_t (&row)[N], int a, 
     for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        r[j].x[2 * k] = half_lo(w[j][k >> 1][k & 1]);
-        r[j].x[2 * k + 1] = half_hi(w[j][k >> 1][k & 1]);
+        const uint32_t h = w[j][k >> 1][k & 1];
+        r[j].x[2 * k] = BITS ? __uint_as_float(h & 0xFFFFu) : half_lo(h);
+        r[j].x[2 * k + 1] = BITS ? __uint_as_float(h >> 16) : half_hi(h);
       }
   } else {
     const auto s = (const __attribute__((address_space(1))) float*)src;
@@ -3498,9 +3500,15 @@ DEV float max16(float m) {  // over the row's sixteen lanes
   m = fmaxf(m, dpp<DPP_ROW_HALF_MIRROR>(m));
   return fmaxf(m, dpp<DPP_ROW_MIRROR>(m));
 }
-// The stored form of a row: fp16 or fp32 values, or the I8_REF codes (and scale).
+DEV void row_of_bits(Row8& r) {  // the values of a row of fp16 bits
+#pragma unroll
+  for (int k = 0; k < 8; ++k) r.x[k] = h2f((uint16_t)__float_as_uint(r.x[k]));
+}
+// The stored form of a row: fp16 (bits: r holds those of fp16 rows of 128 dims, stored
+// as they are, where a conversion would quiet a NaN) or fp32 values, or the I8_REF codes
+// (and scale).
 template <int KV>
-DEV void row_codes(const Row8& r, uint32_t (&w)[8], float& scale) {
+DEV void row_codes(const Row8& r, bool bits, uint32_t (&w)[8], float& scale) {
   if constexpr (KV == KV_I8_REF) {
     float m = fabsf(r.x[0]);  // (a row of 128 NaN has the scale NaN, as append_token gives it)
 #pragma unroll
@@ -3512,7 +3520,7 @@ DEV void row_codes(const Row8& r, uint32_t (&w)[8], float& scale) {
     for (int k = 0; k < 8; ++k) w[k] = (uint32_t)(uint8_t)(int8_t)(int)(r.x[k] * inv);
   } else {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) w[k] = KV == KV_F16 ? (uint32_t)f2h(r.x[k]) : __float_as_uint(r.x[k]);
+    for (int k = 0; k < 8; ++k) w[k] = KV == KV_F16 && !bits ? (uint32_t)f2h(r.x[k]) : __float_as_uint(r.x[k]);
   }
 }
 template <int ESZ>
@@ -3565,14 +3573,19 @@ DEV void append_rows(const AppendParams& P, int id) {
       const TokenIn t = token_in(P, n), t1 = token_in(P, n1), t0 = token_in(P, n0);
       Row8 r[2];
       const int64_t rows[2] = {row * io, (more ? row + nh : row) * io};
-      load_rows8<2>(src, dtype, rows, a, b, in, r);
+      load_rows8<2, KV == KV_F16>(src, dtype, rows, a, b, in, r);
       // (new tokens of a batch's sequences, whose slots come from the table, go one by one)
       const int64_t slot = tok ? token_slot_of(P, t, token_entry(P, n, t)) : -1, next = token_slot_of(P, t1, -1),
                     prev = token_slot_of(P, t0, -1);
       uint32_t w[8], w2[8];
       float sc = 0.f, sc2 = 0.f;
-      row_codes<KV>(r[0], w, sc);
-      row_codes<KV>(r[1], w2, sc2);
+      const bool bits = KV == KV_F16 && dtype == DT_F16;
+      if (bits && io < HD) {
+        row_of_bits(r[0]);
+        row_of_bits(r[1]);
+      }
+      row_codes<KV>(r[0], bits && io == HD, w, sc);
+      row_codes<KV>(r[1], bits && io == HD, w2, sc2);
       const bool pair = (slot & 1) == 0 && more && next == slot + 1;
       if (slot < 0 || i >= D / 8 || ((slot & 1) == 1 && n > 0 && prev == slot - 1)) return;
       const int64_t tix = slot / BS * Hkv + h;
@@ -3604,7 +3617,7 @@ DEV void append_rows(const AppendParams& P, int id) {
   int64_t rows[RB];
 #pragma unroll
   for (int k = 0; k < RB; ++k) rows[k] = ((int64_t)n * nh + min(h + k, nh - 1)) * io;
-  load_rows8<RB>(src, dtype, rows, a, b, in, r);
+  load_rows8<RB, KV == KV_F16>(src, dtype, rows, a, b, in, r);
   bool rot = false;
   float4 t0, t1;
   if (P.rope != ROPE_NONE) {
@@ -3614,6 +3627,11 @@ DEV void append_rows(const AppendParams& P, int id) {
     const float* cs = P.cos_sin + (int64_t)(rot ? pos : 0) * io;
     t0 = *reinterpret_cast<const float4*>(cs + (in ? (half ? 2 * a : a) : 0));
     t1 = *reinterpret_cast<const float4*>(cs + (in ? (half ? 2 * a + 4 : b) : 0));
+  }
+  const bool bits = KV == KV_F16 && dtype == DT_F16 && !is_q && P.rope == ROPE_NONE && io == HD;
+  if (KV == KV_F16 && dtype == DT_F16 && !bits) {
+#pragma unroll
+    for (int k = 0; k < RB; ++k) row_of_bits(r[k]);
   }
   if (P.rope != ROPE_NONE) {
     if (rot && in) {  // (the padding stays +0)
@@ -3643,7 +3661,7 @@ DEV void append_rows(const AppendParams& P, int id) {
   if constexpr (KV != KV_I8_BLK) {
     uint32_t w[8];
     float sc = 0.f;
-    row_codes<KV>(r[0], w, sc);
+    row_codes<KV>(r[0], bits, w, sc);
     const int64_t slot = tok ? token_slot_of(P, tk_in, token_entry(P, n, tk_in)) : -1;
     if (slot < 0 || i >= D / 8) return;
     const int64_t t = slot / BS * Hkv + h;
@@ -3669,6 +3687,16 @@ DEV void append_token(const AppendParams& P, int n, int h) {
   uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
   const int64_t t = slot / BS * P.g.n_kv_heads + h;
   const int o = (int)(slot % BS), d0 = 2 * lane_id(), D = P.g.head_dim;
+  if constexpr (KV == KV_F16) {  // (row_codes: bits)
+    if (P.in_dtype == DT_F16 && P.g.io_hd == HD && (is_v || P.rope == ROPE_NONE)) {
+      const auto* src = reinterpret_cast<const uint16_t*>(is_v ? P.v : P.k) + ((int64_t)n * P.g.n_kv_heads + h) * HD + d0;
+      uint8_t* tile = L + (is_v ? P.g.v_off : P.g.k_off) + (uint64_t)t * P.g.tile_bytes;
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        store1<2>(tile + (is_v ? tile_elem<true>(o, d0 + e, 2, HD) : tile_elem<false>(o, d0 + e, 2, HD)), src[e]);
+      return;
+    }
+  }
   float x0, x1;
   load_kv(P, is_v ? P.v : P.k, is_v, n, h, x0, x1);
   float inv = 0.f;
