@@ -172,3 +172,23 @@ def test_append_f16_bits(ctx):
             for key in ("v",) if rope else ("k", "v"):
                 ref = bits[np.frombuffer(getattr(at, key).tobytes(), np.float16).astype(np.int64)]
                 assert np.array_equal(got[key].view(np.uint16), ref), key
+
+
+def test_append_of_more_threads_than_a_grid_dimension(ctx):
+    """17 M padding tokens and three real ones at the end: 34 M workgroups of 128 threads, where HIP
+    takes less than 2^32 threads in one dimension of a grid."""
+    kv, hkv, hd, n = O.F16, 8, 8, 17_000_000
+    print(f"append of {n} tokens", flush=True)
+    slots = np.full(n, -1, np.int64)
+    slots[-3:] = [BS + 4, BS + 5, 7]
+    r = np.random.default_rng(4400)
+    tail = r.standard_normal((3, hkv, hd)).astype(np.float16)
+    rows_in = ctx.alloc(n * hkv * hd * 2)  # (padding rows are read as they are and not stored)
+    rows_in.upload(tail, (n - 3) * hkv * hd * 2)
+    pool = velokv.Pool(ctx, 1, 2, BS, hkv, hd, kv)
+    ctx.append(pool, 0, rows_in, rows_in, velokv.DT_F16, ctx.upload(slots), n)
+    ctx.sync()
+    ref = O.Layer(2, hkv, BS, 64, kv)
+    x = np.pad(tail, ((0, 0), (0, 0), (0, 64 - hd)))
+    O.append(ref, x, x, slots[-3:])
+    assert_layer_equal(pool, 0, ref)

@@ -634,7 +634,14 @@ int launch_append(const vk_ctx* ctx, const vk_pool* pool, AppendParams& p, void*
   if (runs + rows > 0x7FFFFFFF) return fail(VK_ERR_UNSUPPORTED, "grid too large");
   p.kv_wgs = (int32_t)runs;
   const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
-  return launch(ctx, name.c_str(), dim3((unsigned)(runs + rows)), dim3(128), p, stream);
+  // HIP takes less than 2^32 threads in a dimension of a grid, and launches what is
+  // left of a larger number without an error
+  constexpr int64_t kMaxWgs = 1 << 24;
+  for (int64_t w = 0; w < runs + rows; w += kMaxWgs) {
+    p.wg0 = (int32_t)w;
+    if (int rc = launch(ctx, name.c_str(), dim3((unsigned)std::min(kMaxWgs, runs + rows - w)), dim3(128), p, stream)) return rc;
+  }
+  return VK_OK;
 }
 }  // namespace
 

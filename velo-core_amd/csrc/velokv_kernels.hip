@@ -3722,9 +3722,10 @@ DEV void append_token(const AppendParams& P, int n, int h) {
 // the 16 tokens' tile offsets fold into the instructions; vk_append_kv3 / _d64).
 template <int KV, int D = HD>
 DEV void append_kernel(const AppendParams& P) {
+  const int wg = P.wg0 + (int)blockIdx.x;
   if constexpr (KV == KV_I8_BLK) {
-    if ((int)blockIdx.x < P.kv_wgs) {
-      const int h = (int)blockIdx.x % P.g.n_kv_heads, w0 = (int)blockIdx.x / P.g.n_kv_heads * P.tok_per_wg;
+    if (wg < P.kv_wgs) {
+      const int h = wg % P.g.n_kv_heads, w0 = wg / P.g.n_kv_heads * P.tok_per_wg;
       uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
       if (threadIdx.x >= WAVE)
         append_blk<true, D>(P, P.v, L + P.g.v_off, reinterpret_cast<uint16_t*>(L + P.g.vs_off), w0, P.tok_per_wg, h);
@@ -3732,11 +3733,11 @@ DEV void append_kernel(const AppendParams& P) {
         append_blk<false, D>(P, P.k, L + P.g.k_off, reinterpret_cast<uint16_t*>(L + P.g.ks_off), w0, P.tok_per_wg, h);
       return;
     }
-  } else if ((int)blockIdx.x < P.kv_wgs) {
-    append_token<KV>(P, (int)blockIdx.x / P.g.n_kv_heads, (int)blockIdx.x % P.g.n_kv_heads);
+  } else if (wg < P.kv_wgs) {
+    append_token<KV>(P, wg / P.g.n_kv_heads, wg % P.g.n_kv_heads);
     return;
   }
-  const int id = (int)blockIdx.x - P.kv_wgs;
+  const int id = wg - P.kv_wgs;
   append_rows<KV, row_batch(KV)>(P, id);
 }
 

@@ -74,6 +74,7 @@ struct AppendParams {
   int32_t q_dtype;
   int32_t tok_per_wg;       // I8_BLK: tokens per workgroup (1..64)
   int32_t kv_wgs;           // workgroups of the I8_BLK runs, or of a token and KV head each (small calls)
+  int32_t wg0;              // the launch's first workgroup (0 unless the call takes several launches)
   int32_t row_groups;       // row groups per token: query heads, row_batch of them each; K and V heads (not I8_BLK)
   uint32_t* err;            // the context's misuse word
   unsigned long long* claim;// I8_BLK: [n_blocks] (epoch << 32 | first token) of the last run per block
