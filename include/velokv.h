@@ -329,7 +329,9 @@ typedef struct vk_decode_args {
                                  max_context_len are computed whatever it says */
 } vk_decode_args;
 
-/* Bytes of workspace vk_paged_decode needs for these arguments. */
+/* Bytes of workspace vk_paged_decode needs for these arguments. Small batches may run
+ * in partitions of a workgroup each; with a smaller buffer, which the plan of larger
+ * batches fits, they take that. */
 int vk_paged_decode_workspace(const vk_pool* pool, const vk_decode_args* a, uint64_t* bytes);
 
 /* Name of the attention kernel vk_paged_decode would launch for these arguments

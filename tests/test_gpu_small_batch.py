@@ -140,6 +140,32 @@ def test_append_of_one_sequence_twice(ctx, kv, first):
     close(out.download(q.shape, np.float32), O.paged_decode(ref, q, bt, lens), kv, np.float16)
 
 
+@pytest.mark.parametrize("kv,G", [(O.F16, 4), (O.F16, 7), (O.F32, 4), (O.I8_BLK, 4)])
+def test_scratch_of_the_larger_plan(ctx, kv, G):
+    """A uniform batch in partitions, with a buffer that only fixed partitions fit: it takes those.
+    One byte less is refused."""
+    print(f"small scratch kv={kv} G={G}", flush=True)
+    case = make_case(kv, [1500, 1500], n_kv_heads=2, n_heads=2 * G, seed=3600)
+    pool, layer = gpu_pool(ctx, case), oracle_layer(case)
+    ref = O.paged_decode(layer, case.q, case.block_tables, case.ctx_lens)
+    q, tab, cl = ctx.upload(case.q), ctx.upload(case.block_tables), ctx.upload(case.ctx_lens)
+    stride, args = case.block_tables.shape[1], (case.S, case.n_heads, 1500)
+    assert plan(ctx, pool, case, np.float16)["max_partitions"] > 1
+    need = ctx.decode_workspace_bytes(pool, *args, stride, sum_context_len=3000)
+    ctx.set_decode_schedule(velokv.SCHED_SPLIT)
+    less = ctx.decode_workspace_bytes(pool, *args, stride, sum_context_len=3000)
+    ctx.set_decode_schedule(velokv.SCHED_AUTO)
+    out = ctx.alloc(case.q.size * 4)
+    run = lambda size: ctx.paged_decode(pool, 0, q, velokv.DT_F16, out, cl, *args, block_tables=tab, bt_stride=stride,
+                                        workspace=ctx.alloc(max(need, less)), workspace_bytes=size, sum_context_len=3000)
+    for size in {need, less}:
+        run(size)
+        ctx.sync()
+        close(out.download(case.q.shape, np.float32), ref, kv, np.float16)
+    with pytest.raises(velokv._capi.VkError):
+        run(min(need, less) - 1)
+
+
 # one long context among many short ones: KV heads, lengths
 SKEWED = [(8, [20000] + [200] * 39), (8, [10000] + [150] * 69), (8, [5000] + [60] * 199), (2, [40000] + [200] * 99)]
 

@@ -760,6 +760,19 @@ int split_workspace(vk_ctx* ctx, void* given, uint64_t given_bytes, uint64_t nee
   return VK_OK;
 }
 
+// Whether a call can have `need` bytes of scratch: in the buffer given, or in the
+// context's own, which may grow unless the stream is being captured.
+bool scratch_at_hand(vk_ctx* ctx, const void* given, uint64_t given_bytes, uint64_t need, void* stream) {
+  if (given) return given_bytes >= need;
+  {
+    std::lock_guard<std::mutex> lk(ctx->ws_mu);
+    if (ctx->ws_bytes >= need) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return !stream || (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &st) == hipSuccess &&
+                     st == hipStreamCaptureStatusNone);
+}
+
 constexpr int kPkMaxSeqs = 256;  // sequences a vk_decode_pk_* workgroup ranks
 constexpr int kPkMaxRounds = 16; // items per vk_decode_pk_* workgroup
 
@@ -826,7 +839,8 @@ int wg_fills(const vk_decode_args* a, const vk_pool_desc& d, int64_t waves) {
   return pairs > 0 && pairs * nw >= waves && (nb + nw - 1) / nw <= kMaxPartTokens / kBS && pairs <= 0x7FFFFFFF ? nw : 0;
 }
 
-int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, DecodePlan* pl) {
+// small: the plans of small batches may be taken (in partitions they need other scratch).
+int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, DecodePlan* pl, bool small = true) {
   if (!a) return fail(VK_ERR_BAD_ARG, "args is null");
   const vk_pool_desc& d = pool->desc;
   if (a->layer < 0 || a->layer >= d.n_layer) return fail(VK_ERR_BAD_ARG, "layer %d out of range", a->layer);
@@ -867,7 +881,7 @@ int plan_decode(vk_ctx* ctx, const vk_pool* pool, const vk_decode_args* a, Decod
   const std::string wg = decode_wg_name(d.kv_type, G, a->q_dtype, d64);
   const WgResident wg_res = ctx ? wg_resident_waves(ctx, wg) : WgResident{2048, 2048, 2048, 2048};
   const int64_t wg_waves = wg_res[3];
-  if (sched == VK_SCHED_AUTO && !valu && P == 0 && G <= kMaxGroupTile &&
+  if (small && sched == VK_SCHED_AUTO && !valu && P == 0 && G <= kMaxGroupTile &&
       small_plan(a, d, wg_res, pool->geom.tile_bytes, &waves, &part)) {
     const int64_t nb = ((int64_t)a->max_context_len + kBS - 1) / kBS;
     pl->stream_k = false;
@@ -1093,16 +1107,26 @@ int run_decode(vk_ctx* ctx, vk_pool* pool, const vk_decode_args* a, void* stream
   // sequence's last block appends the token before loading it); every other plan
   // appends in a launch of its own first
   const int kvt = pool->desc.kv_type;
+  const auto folds_rope = [&] { return k_new && rope.style != ROPE_NONE && plan_folds_rope(pool, a, pl); };
+  const auto q_copy_bytes = [&]() -> uint64_t {
+    return rope.style != ROPE_NONE && !folds_rope()
+               ? align_up((uint64_t)a->n_seqs * a->n_heads * pool->geom.io_hd * (a->q_dtype == VK_DT_F32 ? 4 : 2), 256) : 0;
+  };
+  const auto scratch = [&] { return pl.acc_bytes + pl.ml_bytes + pl.prefix_bytes + q_copy_bytes(); };
+  // a small batch's partitions only where their scratch is at hand: else the plan of
+  // larger batches where it takes less
+  if (const uint64_t need = scratch(); pl.wg_waves && pl.max_parts > 1 &&
+                                       !scratch_at_hand(ctx, a->workspace, a->workspace_bytes, need, stream)) {
+    const DecodePlan parts = pl;
+    if ((rc = plan_decode(ctx, pool, a, &pl, false))) return rc;
+    if (scratch() >= need) pl = parts;
+  }
   const bool fold = k_new && plan_folds_append(pool, a, pl);
-  const bool rope_fold = fold && rope.style != ROPE_NONE && plan_folds_rope(pool, a, pl);
+  const bool rope_fold = folds_rope();
   const std::string kernel = rope_fold ? pl.kernel + kRopeSuffix : pl.kernel;
   const bool rope_copy = rope.style != ROPE_NONE && !rope_fold;
-  const uint64_t q_bytes = rope_copy ? align_up((uint64_t)a->n_seqs * a->n_heads * pool->geom.io_hd *
-                                                (a->q_dtype == VK_DT_F32 ? 4 : 2), 256) : 0;
   uint8_t* ws = nullptr;
-  if ((rc = split_workspace(ctx, a->workspace, a->workspace_bytes,
-                            pl.acc_bytes + pl.ml_bytes + pl.prefix_bytes + q_bytes, &ws)))
-    return rc;
+  if ((rc = split_workspace(ctx, a->workspace, a->workspace_bytes, scratch(), &ws))) return rc;
   void* q_rot = rope_copy ? ws + pl.acc_bytes + pl.ml_bytes + pl.prefix_bytes : nullptr;
   if (k_new && (!fold || rope_copy) &&
       (rc = append_new_tokens(ctx, pool, a, pl, k_new, v_new, in_dtype, stream, rope, q_rot)))
@@ -1396,21 +1420,6 @@ extern "C" int vk_tree_verify_plan(const vk_pool* pool, const vk_tree_args* a, v
   return VK_OK;
 }
 
-namespace {
-// Whether a call can have `need` bytes of scratch: in the caller's buffer, or in
-// the context's own, which may grow unless the stream is being captured.
-bool tree_scratch_at_hand(vk_ctx* ctx, const vk_tree_args* a, uint64_t need, void* stream) {
-  if (a->workspace) return a->workspace_bytes >= need;
-  {
-    std::lock_guard<std::mutex> lk(ctx->ws_mu);
-    if (ctx->ws_bytes >= need) return true;
-  }
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return !stream || (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &st) == hipSuccess &&
-                     st == hipStreamCaptureStatusNone);
-}
-}  // namespace
-
 extern "C" int vk_tree_verify(vk_ctx* ctx, vk_pool* pool, const vk_tree_args* a, void* stream) {
   int rc = check_pool(ctx, pool);
   if (rc) return rc;
@@ -1421,7 +1430,7 @@ extern "C" int vk_tree_verify(vk_ctx* ctx, vk_pool* pool, const vk_tree_args* a,
   if ((rc = set_device(ctx))) return rc;
   // short partitions only where their scratch is at hand: not past the caller's
   // buffer, and no growing of the context's own under capture
-  if (pl.max_parts > 1 && !tree_scratch_at_hand(ctx, a, pl.acc_bytes + pl.ml_bytes, stream) &&
+  if (pl.max_parts > 1 && !scratch_at_hand(ctx, a->workspace, a->workspace_bytes, pl.acc_bytes + pl.ml_bytes, stream) &&
       (rc = plan_tree(ctx, pool, a, &pl, false)))
     return rc;
   uint8_t* ws = nullptr;
