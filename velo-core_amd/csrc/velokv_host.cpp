@@ -633,6 +633,7 @@ int launch_append(const vk_ctx* ctx, const vk_pool* pool, AppendParams& p, void*
   const int64_t rows = ((int64_t)p.n_tok + kRowTokens - 1) / kRowTokens * p.row_groups;
   if (runs + rows > 0x7FFFFFFF) return fail(VK_ERR_UNSUPPORTED, "grid too large");
   p.kv_wgs = (int32_t)runs;
+  p.kv_div = hkv >= 8 ? hkv : (int32_t)std::max<int64_t>(1, runs / hkv);
   const std::string name = append_kernel_name(pool->desc.kv_type, pool->desc.head_dim);
   // HIP takes less than 2^32 threads in a dimension of a grid, and launches what is
   // left of a larger number without an error

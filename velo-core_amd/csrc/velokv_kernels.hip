@@ -1001,14 +1001,15 @@ DEV float div_scale(float x, float s, float y) {
 }
 DEV float blk_clamp(float q) { return fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f); }
 DEV float blk_rne(float x, float s, float y) {
-  const float q = s < __builtin_huge_valf() ? div_scale(x, s, y) : x / s;  // (wave-uniform)
+  const float q = s < __builtin_huge_valf() ? div_scale(x, s, y) : x / s;
   return blk_clamp(q);
 }
 DEV int blk_requant(int c, float s_old, float s_new, float y) { return (int)blk_rne((float)c * s_old, s_new, y); }
 DEV int blk_code(float x, float s_new, float y) { return s_new > 0.f ? (int)blk_rne(x, s_new, y) : 0; }
-// The same by a division of each value, for the append folded into a decode: beside a
-// piece's stages the inverse and the scale test spilled up to five registers more
-// (stream-K with RoPE, 2 to 16 query heads per KV head).
+// The same by a division of each value, where the inverse and the scale test cost more
+// in registers than they save: in the append folded into a decode they spilled up to six
+// vector registers more beside a piece's stages (stream-K with RoPE, 2 to 16 query heads
+// per KV head), in append_blk_run ten scalar ones.
 DEV int blk_requant(int c, float s_old, float s_new) { return (int)blk_clamp((float)c * s_old / s_new); }
 DEV int blk_code(float x, float s_new) { return s_new > 0.f ? (int)blk_clamp(x / s_new) : 0; }
 
@@ -3021,7 +3022,14 @@ DEV int prev_block(const AppendParams& P, int n) {
 // The run that starts at token w0 + j (slot `slot`), for KV head h; ms0 holds
 // the slots of tokens w0 .. w0 + 63 (lane i: token w0 + i, -1 past the end), so
 // the first step of the run's forward scan needs no load.
-constexpr int kRunBatch = 4;
+// Members a step of append_blk_run: two, whose rows' loads overlap, keep the path's
+// scalar registers (3,000 single tokens x 8 heads 44.2 us; four 46.7, eight 58.8).
+constexpr int kRunBatch = 2;
+// Tokens from which a run of consecutive slots goes all at once (append_blk_tile):
+// with 128 dims, 1,024 tokens x 8 heads in two-token runs 14.5 us in order and 16.1 at
+// once, 4,096 in four-token runs 38.4 and 33.5; with 64 dims two-token runs 16.8 and 14.0.
+template <int D>
+constexpr int kTileRun = D == HD ? 4 : 2;
 template <bool IS_V, int D>
 DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int w0, int j,
                         int64_t slot, int64_t ms0, int h) {
@@ -3077,7 +3085,7 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
     uint64_t mem = __builtin_amdgcn_ballot_w64(ms >= 0 && lane < stop);
     const int moff = (int)(ms >= 0 ? ms % BS : 0);
     while (mem != 0) {
-      // up to 8 members: their rows loaded together, then the rule. What does
+      // up to kRunBatch members: their rows loaded together, then the rule. What does
       // not depend on the member before (the absmax and candidate scale, and
       // once the running scales are known the new codes) is computed for all
       // members at once; only the running scale and the placement, with its
@@ -3128,21 +3136,21 @@ DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, 
       int cc[kBatch][2];
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
-        const float s_k = h2f((uint16_t)sn[k]), y = blk_inv(s_k);
-        cc[k][0] = k < nb ? blk_code(xs[k][0], s_k, y) : 0;
-        cc[k][1] = k < nb ? blk_code(xs[k][1], s_k, y) : 0;
+        const float s_k = h2f((uint16_t)sn[k]);
+        cc[k][0] = k < nb ? blk_code(xs[k][0], s_k) : 0;
+        cc[k][1] = k < nb ? blk_code(xs[k][1], s_k) : 0;
       }
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
         if (k < nb) {
           const int o = ok[k];
           if (sn[k] > so[k] && o > 0) {
-            const float s_o = h2f((uint16_t)so[k]), s_k = h2f((uint16_t)sn[k]), y = blk_inv(s_k);
+            const float s_o = h2f((uint16_t)so[k]), s_k = h2f((uint16_t)sn[k]);
 #pragma unroll
             for (int u = 0; u < BS; ++u) {
               if (u < o) {
-                cd[u][0] = blk_requant(cd[u][0], s_o, s_k, y);
-                cd[u][1] = blk_requant(cd[u][1], s_o, s_k, y);
+                cd[u][0] = blk_requant(cd[u][0], s_o, s_k);
+                cd[u][1] = blk_requant(cd[u][1], s_o, s_k);
               }
             }
           }
@@ -3259,7 +3267,8 @@ DEV uint32_t pack_i8x4(float a, float b, float c, float d) {
 // Bound by that and by the vector ALUs (2.4 growths in a fresh block, 45
 // instructions each and lane), where a wave with two dims of every token went
 // through the tokens one after another: 8,000 tokens x 8 heads with 32 rotated
-// query heads 163 -> 53 us (K and V alone 53 -> 29), 2,048 draft tokens 23 -> 22.
+// query heads 163 -> 52 us, 3,000 in long runs (K and V alone) 27.2 -> 16.3, 2,048 draft
+// tokens in runs of eight 18.8 -> 16.6.
 template <bool IS_V, int D>
 DEV void append_blk_tile(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int n0, int m, int o0,
                          int64_t b, int h) {
@@ -3366,6 +3375,15 @@ DEV void append_blk_tile(const AppendParams& P, const void* src, uint8_t* codes,
   if (lane == 0) *sp = (uint16_t)s_prev;
 }
 
+// The kernel's arguments as read again here: the path that takes a block at once reads
+// its own when it is taken. Held beside the in-order path's they spilled 50 scalar
+// registers more, for which single tokens paid too (1,024 x 8 heads 19.2 us when the
+// kernel had one path, 21.7 with two, 17.9 with this, kRunBatch and the plain division).
+DEV AppendParams reload_params() {
+  auto kp = (const __attribute__((address_space(4))) AppendParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(kp));
+  return *kp;
+}
 // The runs that start inside tokens [w0, w0 + T) of the call, in order. A token
 // starts a run when it is not padding and the nearest non-padding token before
 // it is in another block (or there is none).
@@ -3401,17 +3419,19 @@ DEV void append_blk(const AppendParams& P, const void* src, uint8_t* codes, uint
     if (claim) old = __hip_atomic_exchange(&P.claim[slot / BS], me, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // tokens in consecutive slots of the block, and nothing of the block after them
     // (the call's end or a token of another block; no padding or reordering within,
-    // and no token that goes on in a block filled to its end): all at once (a half-split
-    // rotation needs its partners in the lanes that path gives them; one token is done
-    // sooner with its dims over the wave, 5.4 us a call against 7.4)
+    // and no token that goes on in a block filled to its end): all at once from kTileRun
+    // tokens (a half-split rotation needs its partners in the lanes that path gives them)
     const int o0 = (int)(slot % BS);
     const uint64_t same = __builtin_amdgcn_ballot_w64(lane >= j && ms64 == slot + (lane - j)) >> j;
     const int m = __builtin_ctzll(~same | (1ull << (BS - o0)));
-    const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m <= BS
-    const int nx = __shfl((int)(ms64 / BS), after != 0 ? j + m + __builtin_ctzll(after) : 0, WAVE);
-    if (m > 1 && (after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok) &&
-        (IS_V || P.rope != ROPE_HALF || P.g.io_hd == D))
-      append_blk_tile<IS_V, D>(P, src, codes, scales, w0 + j, m, o0, slot / BS, h);
+    bool whole = m >= kTileRun<D> && (IS_V || P.rope != ROPE_HALF || P.g.io_hd == D);
+    if (whole) {
+      const uint64_t after = (__builtin_amdgcn_ballot_w64(ms64 >= 0) >> j) >> m;  // m <= BS
+      const int nx = __shfl((int)(ms64 / BS), after != 0 ? j + m + __builtin_ctzll(after) : 0, WAVE);
+      whole = after != 0 ? nx != (int)(slot / BS) : w0 + WAVE >= P.n_tok;
+    }
+    if (whole)
+      append_blk_tile<IS_V, D>(reload_params(), src, codes, scales, w0 + j, m, o0, slot / BS, h);
     else
       append_blk_run<IS_V, D>(P, src, codes, scales, w0, j, slot, ms64, h);
     if (claim && (uint32_t)(old >> 32) == P.epoch && old != me) flag_misuse(P.err, MISUSE_BLK_SPLIT_RUN);
@@ -3725,7 +3745,13 @@ DEV void append_kernel(const AppendParams& P) {
   const int wg = P.wg0 + (int)blockIdx.x;
   if constexpr (KV == KV_I8_BLK) {
     if (wg < P.kv_wgs) {
-      const int h = wg % P.g.n_kv_heads, w0 = wg / P.g.n_kv_heads * P.tok_per_wg;
+      // heads or windows fastest (AppendParams::kv_div): a window's heads side by side use
+      // all XCDs whatever windows have runs (eight heads and up); with fewer heads they
+      // would not (739 tokens x 2 heads in two-token runs, half the windows: 8.3 us, 7.2
+      // with a head's windows side by side)
+      const int a = wg / P.kv_div, b = wg - a * P.kv_div;
+      const bool heads = P.kv_div == P.g.n_kv_heads;
+      const int h = heads ? b : a, w0 = (heads ? a : b) * P.tok_per_wg;
       uint8_t* L = P.base + (uint64_t)P.layer * P.g.layer_stride;
       if (threadIdx.x >= WAVE)
         append_blk<true, D>(P, P.v, L + P.g.v_off, reinterpret_cast<uint16_t*>(L + P.g.vs_off), w0, P.tok_per_wg, h);

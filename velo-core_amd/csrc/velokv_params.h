@@ -50,11 +50,12 @@ enum RopeStyle : int32_t { ROPE_NONE = 0, ROPE_INTERLEAVED = 1, ROPE_HALF = 2 };
 // VK_MISUSE_*); the kernels still run to completion on the clamped input.
 enum Misuse : uint32_t { MISUSE_PAGE_OUT_OF_POOL = 1u, MISUSE_BLK_SPLIT_RUN = 2u };
 
-// Append of n_tok tokens, workgroups of two waves: kv_wgs = ceil(n_tok / T) Hkv of
-// them (I8_BLK pools, else 0; T = tok_per_wg) write K (wave 0) and V (wave 1) of a
-// KV head and the runs that start in a window of T tokens; ceil(n_tok / 8)
-// row_groups follow for the rows that are stored one by one: query heads to
-// rotate, and K and V of the other pool types.
+// Append of n_tok tokens, workgroups of two waves (K and V of a KV head, or two groups
+// of four tokens): first kv_wgs of them, over I8_BLK pools ceil(n_tok / T) Hkv, T =
+// tok_per_wg, each for the runs that start in a window of T tokens; over the others
+// n_tok Hkv, one token each, in small calls and else none. ceil(n_tok / 8) row_groups
+// follow for the rows that are stored one by one: query heads to rotate, and where
+// kv_wgs is 0 K and V.
 struct AppendParams {
   uint8_t* base;            // pool base (all layers)
   PoolGeom g;
@@ -72,8 +73,9 @@ struct AppendParams {
   void* q;                  // [n_tok][n_heads][D] of q_dtype, rotated in place unless q_out is given
   void* q_out;              // or the rotated rows go here (same shape and type), q left unchanged
   int32_t q_dtype;
-  int32_t tok_per_wg;       // I8_BLK: tokens per workgroup (1..64)
+  int32_t tok_per_wg;       // I8_BLK: tokens per workgroup (1..16)
   int32_t kv_wgs;           // workgroups of the I8_BLK runs, or of a token and KV head each (small calls)
+  int32_t kv_div;           // I8_BLK runs: n_kv_heads (workgroups of a window side by side) or the windows (of a head)
   int32_t wg0;              // the launch's first workgroup (0 unless the call takes several launches)
   int32_t row_groups;       // row groups per token: query heads, row_batch of them each; K and V heads (not I8_BLK)
   uint32_t* err;            // the context's misuse word
