@@ -1,5 +1,6 @@
 // Sweep of the small-batch plan rule (velokv_plan.h small_plan) over batch shapes,
-// length sums (true, unknown, too small) and kernels' resident waves.
+// length sums (true, unknown, too small) and kernels' resident waves; its choices and
+// tree_short_part's at measured calls.
 #include <cstdio>
 #include <cstring>
 
@@ -85,7 +86,32 @@ static void check_skewed(const Skewed& c) {
            c.longest, c.rest, !c.small, c.us, c.sk_us);
 }
 
+// Tree calls: `pairs` units a partition of row_tiles tiles, on 1,024 SIMDs; measured us of partitions
+// of 64, 96, 128, 192 and 256 tokens. The rule's choice is within 7 % of the best, and of 256 at most 2 % above.
+struct Tree { int kv; int64_t tokens, pairs; int row_tiles; double us[5]; };
+static const Tree kTree[] = {
+    {VK_KV_I8_BLK, 508, 1, 1, {9.2, 10.3, 11.5, 13.2, 15.4}},     {VK_KV_I8_BLK, 4008, 1, 1, {14.2, 14.2, 13.8, 15.0, 16.4}},
+    {VK_KV_I8_BLK, 8008, 1, 1, {22.5, 18.6, 17.0, 17.4, 18.1}},   {VK_KV_I8_BLK, 16008, 1, 1, {39.6, 28.2, 24.5, 22.4, 21.6}},
+    {VK_KV_I8_BLK, 8008, 8, 2, {24.5, 20.7, 19.6, 21.4, 22.7}},   {VK_KV_I8_REF, 6009, 8, 1, {19.0, 16.1, 15.5, 15.1, 16.4}},
+    {VK_KV_F16, 6013, 10, 1, {21.9, 18.1, 17.1, 17.2, 17.6}},     {VK_KV_F16, 16009, 8, 1, {42.5, 34.0, 28.3, 24.9, 21.8}},
+    {VK_KV_F16, 2008, 8, 2, {13.9, 15.0, 15.6, 19.3, 21.8}},      {VK_KV_F32, 4008, 8, 2, {28.0, 30.8, 34.6, 45.0, 55.4}},
+    {VK_KV_F32, 16009, 8, 1, {59.5, 52.8, 40.1, 38.2, 40.7}},
+};
+
+static void check_tree(const Tree& c) {
+  static const int parts[5] = {64, 96, 128, 192, 256};
+  const int got = tree_short_part(c.tokens, c.pairs, 1024, c.row_tiles, c.kv);
+  double us = 1e9, best = 1e9;
+  for (int i = 0; i < 5; ++i) {
+    if (parts[i] == got) us = c.us[i];
+    if (c.us[i] < best) best = c.us[i];
+  }
+  if (us <= 1.07 * best && us <= 1.02 * c.us[4]) return;
+  if (bad++ < 10) printf("tree: kv %d, %lld tokens: %d, %.1f us, best %.1f\n", c.kv, (long long)c.tokens, got, us, best);
+}
+
 int main() {
+  for (const Tree& c : kTree) check_tree(c);
   for (const Skewed& c : kSkewed) check_skewed(c);
   for (int64_t resident : {1024, 2048, 4096, 8192})
     for (int kv : {VK_KV_F32, VK_KV_F16, VK_KV_I8_REF, VK_KV_I8_BLK})

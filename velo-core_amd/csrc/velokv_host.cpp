@@ -1291,9 +1291,7 @@ struct TreePlan {
   std::string kernel, pfx_kernel;
 };
 
-// The least partitions of a tree call of few units, in tokens, and the waves per CU
-// up to which they are taken (plan_tree).
-constexpr int kTreeShort[] = {64, 96, 128, 192};
+// Waves per CU up to which tree calls take short partitions (tree_short_part).
 constexpr int64_t kTreeShortWaves = 4;
 
 // short_parts: partitions of less than 256 tokens may be taken (they need more scratch).
@@ -1369,19 +1367,12 @@ int plan_tree(vk_ctx* ctx, const vk_pool* pool, const vk_tree_args* a, TreePlan*
     P = kMaxPartTokens;
     for (int c = 256; c < kMaxPartTokens; c *= 2)
       if (pairs * ((tokens + c - 1) / c) <= 4 * waves) { P = c; break; }
-    // Calls whose units leave SIMDs empty take shorter ones, the shortest whose
-    // units are at most one wave per SIMD: a wave walks its blocks one after
-    // another (about 1.2 us a block over fp16, 2.6 over fp32), and past one wave
-    // per SIMD the merge and its partials cost more than the walk saves. 64 / 256
-    // tokens at 8 nodes: 1,500 int8 tokens, 4 units a partition, 9.7 / 15.1 us;
-    // 4,000 fp32 tokens, 16 units, 18.6 / 33.7. Past the line, 192 / 256: 512 units
-    // a partition, 4,000 int8 tokens, 99.8 / 95.3; 192 units, 1,500 fp16 tokens,
-    // 44.0 / 32.1. A call that one 256-token partition covers stays whole: it needs
-    // no scratch, so such calls on several streams share nothing.
+    // Calls whose units leave SIMDs empty take shorter ones. A call that one 256-token
+    // partition covers stays whole: it needs no scratch, so such calls on several streams
+    // share nothing.
     const int64_t simds = std::min(waves, kTreeShortWaves * (ctx ? ctx->n_cu : 256));
     if (short_parts && P == 256 && tokens > 256 && pl->prefix_chunks == 0)
-      for (int c : kTreeShort)
-        if (pairs * ((tokens + c - 1) / c) <= simds) { P = c; break; }
+      P = tree_short_part(tokens, pairs, simds, pl->rt, d.kv_type);
   }
   pl->part_tokens = P;
   pl->max_parts = pl->prefix_chunks + (int32_t)std::max<int64_t>(1, (tokens + P - 1) / P);

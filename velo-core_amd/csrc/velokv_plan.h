@@ -154,4 +154,32 @@ inline bool small_plan(const vk_decode_args* a, const vk_pool_desc& d, const WgR
   return (*part_blocks + nw - 1) / nw <= kMaxPartTokens / kBS;
 }
 
+// Partition of a tree call of few units (`pairs` a partition), in tokens: of 64, 96, 128,
+// 192 and 256 that whose longest walk and merge take least. A wave walks its blocks one
+// after another (kTreeBlockNs, by row tiles of 16 per unit and KV type) and the merge
+// reads a row's partials eight at a time (kTreePartialNs each): one sequence, 8 nodes,
+// one KV head, int8 blocks, 64 / 256 tokens: 500 tokens 9.2 / 15.4 us, 4,000 14.2 / 16.4
+// (128: 13.8), 16,000 39.6 / 21.6; fp32 8,000 25.2 / 35.8. Below 256 only while the units
+// are at most `simds`: past one wave per SIMD the partials cost more than the walk saves
+// (192 / 256: 512 units a partition, 4,000 int8 tokens, 99.8 / 95.3; 192 units, 1,500
+// fp16 tokens, 44.0 / 32.1).
+constexpr int64_t kTreePartialNs = 110;
+inline int64_t tree_block_ns(int kv_type, int row_tiles) {
+  const bool one = row_tiles == 1;
+  switch (kv_type) {
+    case VK_KV_F32: return one ? 1600 : 2750;
+    case VK_KV_F16: return one ? 500 : 840;
+    default: return one ? 520 : 760;
+  }
+}
+inline int tree_short_part(int64_t tokens, int64_t pairs, int64_t simds, int row_tiles, int kv_type) {
+  const auto ns = [&](int part) {
+    return tree_block_ns(kv_type, row_tiles) * (part / kBS) + kTreePartialNs * ((tokens + part - 1) / part);
+  };
+  int best = 256;
+  for (int part : {64, 96, 128, 192})
+    if (pairs * ((tokens + part - 1) / part) <= simds && ns(part) < ns(best)) best = part;
+  return best;
+}
+
 }  // namespace velokv
