@@ -177,8 +177,9 @@ int vk_ctx_set_decode_kernel(vk_ctx* ctx, int kind);
  * unless vk_decode_args.sum_context_len says the batch is uniform, or the VALU
  * family was requested; a small batch whose lengths' sum is known, or of one
  * sequence, runs the workgroup split, one workgroup per (sequence, KV head), or
- * per partition of the longer contexts with a merge launch). A nonzero partition_tokens always uses fixed partitions. No
- * reference counterpart. */
+ * per partition of the longer contexts with a merge launch, except where one long
+ * context among short ones or a uniform batch's shape makes the others faster). A
+ * nonzero partition_tokens always uses fixed partitions. No reference counterpart. */
 #define VK_SCHED_AUTO 0
 #define VK_SCHED_SPLIT 1
 #define VK_SCHED_STREAM 2
@@ -452,7 +453,7 @@ typedef struct vk_tree_args {
 } vk_tree_args;
 
 /* Bytes of split-K workspace vk_tree_verify needs for these arguments (0 when
- * one partition covers every sequence). Calls of few units take partitions of less
+ * one partition covers every sequence). Calls of few units may take partitions of less
  * than 256 tokens; with a smaller buffer, which 256-token ones fit, they take those. */
 int vk_tree_verify_workspace(const vk_pool* pool, const vk_tree_args* a, uint64_t* bytes);
 

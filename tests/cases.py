@@ -80,7 +80,7 @@ def oracle_layer(case: Case, with_last=True):
 
 
 def tol_check(got, ref, atol=2e-3, rtol=1e-2):
-    """The north-star tolerance: |got - ref| <= atol + rtol * |ref| elementwise."""
+    """The stated tolerance: |got - ref| <= atol + rtol * |ref| elementwise."""
     err = np.abs(got.astype(np.float64) - ref.astype(np.float64))
     bound = atol + rtol * np.abs(ref.astype(np.float64))
     bad = err > bound

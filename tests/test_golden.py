@@ -1,7 +1,7 @@
 """Configuration-1 known answers committed under tests/golden/ (written by
 tests/golden/make_golden.py): the oracle must keep reproducing them on the CPU,
 and the HIP path must match them (bit-exact pool bytes, decode within the
-north-star tolerance) on the GPU."""
+stated tolerance) on the GPU."""
 import hashlib
 import os
 

@@ -4,7 +4,7 @@ the attention kernel per layer): the append kernel with the slots derived from
 the block table in the kernel, then the decode, over every schedule.
 Each case is checked three ways: pool bytes bit for bit against the oracle's
 append of the same tokens and against vk_append + vk_paged_decode (same
-schedule) on a second pool, and outputs within the north-star tolerance of the
+schedule) on a second pool, and outputs within the stated tolerance of the
 oracle's decode. Under stream-K the two calls cut the contexts into the same
 pieces, so their outputs are also compared bit for bit; under the workgroup
 split the folding wave's range is kFoldBlocks shorter, so outputs agree to fp32

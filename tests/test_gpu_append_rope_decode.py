@@ -6,7 +6,7 @@ kernels.metal:103-131 is the reference's rotation.
 
 Checked against the oracle's fused RoPE append at those positions (the same
 table) followed by its decode: pool bytes bit for bit, outputs within the
-north-star tolerance; and against the two-call path on a second pool
+stated tolerance; and against the two-call path on a second pool
 (vk_append_rope writing the rotated q, then vk_paged_decode under the same
 schedule): pool bytes bit for bit, and under stream-K, where both calls cut the
 contexts into the same pieces and round the rotated q the same way, outputs bit

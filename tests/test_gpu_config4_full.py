@@ -10,7 +10,7 @@ appended, an 8-node 2-2-2 tree verified with the shared prefix declared
 Checked against the oracle on one layer:
   - the pool bytes after the appends and copies, then after the commit, bit
     for bit (the oracle performs the same appends, copies and commits);
-  - the verify outputs of 8 sampled sequences within the north-star
+  - the verify outputs of 8 sampled sequences within the stated
     tolerance (the oracle's vko_tree_verify restricted to their table rows).
 Tree semantics as vk_tree_verify defines them (node j at context_len + j, a
 node sees its ancestors and itself); kernels.metal:512-599 is the reference's

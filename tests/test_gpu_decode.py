@@ -1,4 +1,4 @@
-"""GPU parity of paged decode attention against the oracle, within the north-star
+"""GPU parity of paged decode attention against the oracle, within the stated
 tolerance (|err| <= 2e-3 + 1e-2 |ref|, fp32-accumulated oracle), for every KV
 type, query dtype, GQA group size and split-K partition size."""
 import numpy as np
@@ -293,7 +293,7 @@ def test_decode_outlier_queries(ctx, sched, kv):
     """q with x10 and x30 outlier channels (|q| up to about 100), as fp16 and as
     fp32: the int8 kernels' biased products, sum_d q (1152 + c) - 1152 sum_d q,
     lose bits in proportion to sum_d |q|, and an fp32 q takes the hi + lo split.
-    Outputs stay within the north-star tolerance of the oracle over the same q,
+    Outputs stay within the stated tolerance of the oracle over the same q,
     on the workgroup split (int8) or split-K (fp16) and on stream-K. One pool
     and one oracle layer serve the four queries."""
     lens = synth.rng(451).integers(1, 3000, 64)

@@ -4,7 +4,7 @@ computes in fp32): decode on every schedule (fixed partitions on the matrix
 cores and on the VALU, stream-K, workgroup split), any GQA group size, and tree
 verify, each against the oracle. With fp32 K, V and q the matrix-core kernels
 (v_mfma_f32_16x16x4f32) keep every operand in fp32, so the bound here is far
-tighter than the north-star tolerance: |err| <= 2e-5 + 2e-4 |ref|."""
+tighter than the stated tolerance: |err| <= 2e-5 + 2e-4 |ref|."""
 import numpy as np
 import pytest
 

@@ -8,7 +8,7 @@ its own and decodes those sequences. So each test checks, at full size:
   - the pool bytes (codes and scales) of the sampled sequences' blocks, bit for
     bit against the oracle's append of the same inputs;
   - the decode of the sampled sequences against the oracle, within the
-    north-star tolerance, for every schedule the planner picks at that shape
+    stated tolerance, for every schedule the planner picks at that shape
     (AUTO) and the ones it can be forced to, with the plan asserted: the
     workgroup split of config 5 walks 256 blocks per wave (all four block-id
     windows), the headline 128.

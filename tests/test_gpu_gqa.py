@@ -4,7 +4,7 @@ Such ratios run the "_gx" matrix-core kernels, which take the group size at run
 time: decode on every schedule (fixed partitions, stream-K, workgroup split,
 vk_append_decode) up to 16 query heads per KV head, fixed partitions with two
 16-row tiles up to 32; tree verify (with and without the shared-prefix pass)
-for any size. Oracle comparison within the north-star tolerance."""
+for any size. Oracle comparison within the stated tolerance."""
 import numpy as np
 import pytest
 

@@ -5,7 +5,7 @@ the 128-dim tiles at D = 64), so it holds and reads its own bytes only.
 
 The pool bytes must equal the oracle's layer built at head_dim 64 (bit for bit,
 every KV type) and attention must equal the oracle's at head_dim 64 (within the
-north-star tolerance). The oracle at 64 dims is pinned on the CPU against the
+stated tolerance). The oracle at 64 dims is pinned on the CPU against the
 oracle at 128 dims over zero-padded rows (tests/test_oracle.py)."""
 import numpy as np
 import pytest

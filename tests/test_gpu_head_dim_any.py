@@ -6,7 +6,7 @@ softmax scale defaults to 1/sqrt(hd).
 
 The pool bytes must equal the oracle's layer at T over the same rows zero-padded
 (bit for bit, every KV type), and attention must equal the oracle's over that
-layer with the 1/sqrt(hd) scale (within the north-star tolerance). That padded
+layer with the 1/sqrt(hd) scale (within the stated tolerance). That padded
 oracle is pinned on the CPU against the reference-kernel restatements at hd
 itself and a numpy closed form of the int8 block rule (tests/test_oracle.py).
 hd = 80 and 40 leave a lane group's last 8-dim chunks of q past the row (the

@@ -1,7 +1,7 @@
 """GPU parity of the packed workgroup split (vk_decode_pk_*: the (sequence, KV
 head) pairs dealt longest first to one workgroup per resident slot in snake
 order, split evenly over the workgroup's waves, split pairs combined in LDS)
-against the oracle, within the north-star tolerance: many pairs per workgroup,
+against the oracle, within the stated tolerance: many pairs per workgroup,
 ties and empty contexts in the ranking, every GQA group, fp16 / INT8 KV, fp16 and
 fp32 queries, and a batch with fewer pairs than workgroups.
 kernels.metal:672-732, 440-501; llama_cpu.rs:251-284."""

@@ -7,7 +7,7 @@ to back (48 tokens: 3 tiles, the page and the tile in it found by division), so 
 % 16 and the pool bytes equal those of a 16-token pool whose tables list the
 pages' tiles. The checks therefore compare against the oracle on the expanded
 16-token tables (bit-exact pool bytes, decode and tree verify within the
-north-star tolerance), and for fp16 / fp32 KV also against the oracle run
+stated tolerance), and for fp16 / fp32 KV also against the oracle run
 directly with the page size (which pins the expansion itself)."""
 import numpy as np
 import pytest

@@ -3,7 +3,7 @@
 full pages aliased, its partial last page copied on write), append their own
 suffixes, and decode over the aliased pages. The GPU pool must equal the
 oracle's byte for byte after the same copies and appends, and the decode must
-match within the north-star tolerance."""
+match within the stated tolerance."""
 import numpy as np
 import pytest
 

@@ -2,7 +2,7 @@
 (sequence, KV head), or partitions of a workgroup each and the merge launch, for
 every KV type, q type and head width, at context lengths around a tile, a
 wave's share and a partition; the append and the rotation folded in for the
-plans that fold them. Pool bytes bit for bit and outputs within the north-star
+plans that fold them. Pool bytes bit for bit and outputs within the stated
 tolerance of the oracle (cases.tol_check; fp32 pools with fp32 q within
 2e-5 + 2e-4 |ref|, the bound of tests/test_gpu_fp32_kv.py)."""
 import numpy as np

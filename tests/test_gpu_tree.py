@@ -1,6 +1,6 @@
 """GPU parity of tree-verify attention against the oracle (vko_tree_verify:
 fp32 two-pass softmax over the committed context plus the mask-selected tree
-nodes), within the north-star tolerance, and the config-4 flow: a shared prefix
+nodes), within the stated tolerance, and the config-4 flow: a shared prefix
 whose pages alias across sequences, copy-on-write of the partial shared block,
 suffix and draft-token appends, then tree verify."""
 import numpy as np
@@ -312,7 +312,7 @@ def test_tree_shared_prefix_bad_arguments(ctx):
         assert e.value.code == velokv.ERR_BAD_ARG
 
 
-# The bound of the fp32-q test, 4-5x tighter than the north-star tolerance
+# The bound of the fp32-q test, 4-5x tighter than the stated tolerance
 # (2e-3 + 1e-2 |ref|); q rounded to fp16 misses it on the test's inputs
 TIGHT = {O.F16: dict(atol=5e-4, rtol=2e-3), O.I8_BLK: dict(atol=5e-4, rtol=2e-3)}
 

@@ -3,7 +3,7 @@ split-K scratch is the library's fixed per-device array) against vk_paged_decode
 through the C ABI: two calls in a row, the second with a smaller input, for the
 stream-K schedule (ragged batches) and fixed split-K partitions, both of which
 keep partials in the scratch; outputs must equal vk_paged_decode's bit for bit
-(same kernels, same schedule) and the oracle's within the north-star tolerance.
+(same kernels, same schedule) and the oracle's within the stated tolerance.
 Also: a caller workspace is refused, and a call whose scratch would exceed the
 array is refused before anything is launched."""
 import numpy as np

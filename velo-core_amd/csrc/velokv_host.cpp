@@ -778,7 +778,7 @@ constexpr int kPkMaxSeqs = 256;  // sequences a vk_decode_pk_* workgroup ranks
 constexpr int kPkMaxRounds = 16; // items per vk_decode_pk_* workgroup
 
 // Blocks' worth of time the append costs the wave that folds it into a
-// workgroup-split decode (vk_append_decode over I8_BLK pools): that wave's range
+// workgroup-split decode (vk_append_decode, plan_folds_append): that wave's range
 // is this much shorter.
 constexpr int kFoldBlocks = 3;
 struct DecodePlan {

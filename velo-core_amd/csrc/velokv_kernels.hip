@@ -1035,8 +1035,8 @@ DEV void blk_put(int (&cd)[BS][2], int o, float& s_old, uint16_t& s_bits, float 
   s_old = s_new;
 }
 
-// ---- the append of vk_append_decode inside the decode launch (I8_BLK; fp16
-// pools under stream-K store the new rows as they are, fold_finish) ----------
+// ---- the append of vk_append_decode inside the decode launch (the rule below is
+// I8_BLK's; the other types store the new rows by their own, fold_finish) ------
 // The piece that holds a sequence's last context token (position ctx - 1)
 // appends the sequence's new K and V rows there before it loads that block: the
 // rule of append_blk_run for a run of one token at offset o = (ctx - 1) % 16
@@ -1199,7 +1199,7 @@ DEV void fold_claim_check(const FoldIn& f, const DecodeParams& P, int s) {
   }
 }
 
-// New row e (0 K, 1 V) of an I8_REF pool by append_ref's rule: fp32 scale
+// New row e (0 K, 1 V) of an I8_REF pool by append_token's rule: fp32 scale
 // amax / 127, codes trunc(x * (127 / amax)).
 template <bool IS_V, int D>
 DEV void fold_ref_row(const FoldIn& f, const DecodeParams& P) {
@@ -1368,7 +1368,7 @@ DEV void attn_piece(const DecodeParams& P, int s, int kvh, int rg, int start, in
   // int8 K enters the score products as fp16 1152 + c (two v_perm per four
   // codes) and the decode subtracts qb = 1152 * sum_d q[row n][d] (of hi + lo
   // when split) from each score; its fp32 sums then carry 1152 sum q, rounded in
-  // proportion to sum |q| (within the north-star tolerance for queries with x30
+  // proportion to sum |q| (within the tests' tolerance for queries with x30
   // outlier channels). Tree verify subtracts 1152 from the codes in fp16 first
   // (exact) and needs no qb: its fp32 queries keep their precision.
   constexpr bool KBIAS = I8 && !TREE;
@@ -2932,8 +2932,9 @@ __device__ void decode_merge_sk(const MergeParams& P) {
 
 // =============================================================================
 // KV append (kernels.metal:619-645 kv_update, 753-802 kv_update_int8).
-// Workgroup (token n, KV head h) with two waves: wave 0 writes K, wave 1 writes V.
-// Lane l owns dims 2l and 2l+1.
+// Workgroups of two waves (AppendParams): over I8_BLK pools wave 0 writes K and wave 1 V
+// of the runs of a window and KV head (append_blk), in small calls of the other types of a
+// token and KV head (append_token), in longer ones rows four tokens a wave (append_rows).
 // =============================================================================
 // RoPE position of token m: the caller's, or without a position array the new
 // token's (context_len - 1, as its slot is derived).
@@ -3004,8 +3005,8 @@ DEV void load_kv(const AppendParams& P, const void* src, bool is_v, int m, int h
 //   if s_new > s_old: c' = clamp(rne((c * s_old) / s_new)) for tokens before offset
 //   c = s_new > 0 ? clamp(rne(x / s_new)) : 0
 // Slots are read 64 tokens at a time (lane j: token base + j) and runs are found
-// with ballots; the K/V rows of up to 8 members are loaded together before the
-// rule runs over them.
+// with ballots; the K/V rows of up to kRunBatch members are loaded together before
+// the rule runs over them.
 
 // Block of the nearest non-padding token before token n of the call, or -1.
 DEV int prev_block(const AppendParams& P, int n) {
@@ -3019,9 +3020,6 @@ DEV int prev_block(const AppendParams& P, int n) {
   return -1;
 }
 
-// The run that starts at token w0 + j (slot `slot`), for KV head h; ms0 holds
-// the slots of tokens w0 .. w0 + 63 (lane i: token w0 + i, -1 past the end), so
-// the first step of the run's forward scan needs no load.
 // Members a step of append_blk_run: two, whose rows' loads overlap, keep the path's
 // scalar registers (3,000 single tokens x 8 heads 44.2 us; four 46.7, eight 58.8).
 constexpr int kRunBatch = 2;
@@ -3030,6 +3028,9 @@ constexpr int kRunBatch = 2;
 // once, 4,096 in four-token runs 38.4 and 33.5; with 64 dims two-token runs 16.8 and 14.0.
 template <int D>
 constexpr int kTileRun = D == HD ? 4 : 2;
+// The run that starts at token w0 + j (slot `slot`), for KV head h; ms0 holds
+// the slots of tokens w0 .. w0 + 63 (lane i: token w0 + i, -1 past the end), so
+// the first step of the run's forward scan needs no load.
 template <bool IS_V, int D>
 DEV void append_blk_run(const AppendParams& P, const void* src, uint8_t* codes, uint16_t* scales, int w0, int j,
                         int64_t slot, int64_t ms0, int h) {
@@ -4252,8 +4253,8 @@ VK_D64_DECODE(0) VK_D64_DECODE(1) VK_D64_DECODE(2) VK_D64_DECODE(3)
   }
 VK_D64_WG(0) VK_D64_WG(1) VK_D64_WG(2) VK_D64_WG(3)
 // vk_append_rope_decode: the kernels that fold the append (stream-K over fp16
-// and I8_BLK pools, the workgroup split over I8_BLK pools), with the new K row
-// and q rotated in registers; suffix _rope
+// and I8_BLK pools, the workgroup split over any pool), with the new K row and q
+// rotated in registers; suffix _rope
 #define VK_ROPE_SK(KV, TAG, QT, D)                                                  \
   extern "C" __global__ void __launch_bounds__(64 * kSkWaves) VK_TWO_WAVES          \
       vk_decode_sk_kv##KV##TAG##_rope(const DecodeParams P) {                       \

@@ -131,7 +131,7 @@ struct DecodeParams {
   int32_t page_tiles;       // page tokens / 16: table entry p holds tiles p * page_tiles .. (p + 1) * page_tiles - 1
   int32_t io_hd;            // head_dim: q / out row length (a multiple of 8 up to 128)
   int32_t tile_hd;          // tile width, 64 or 128 (>= io_hd; the dims past io_hd hold zeros)
-  int32_t max_parts;        // partitions per sequence in the grid
+  int32_t max_parts;        // partitions per sequence in the grid (workgroup split: at most)
   int32_t part_tokens;      // tokens per partition (multiple of the block size)
   int32_t cap_tokens;       // tokens a table row can address: min(max_parts*part_tokens, bt_stride*bs)
   int32_t n_nodes;          // query rows per (sequence, head): 1 for decode
@@ -145,9 +145,9 @@ struct DecodeParams {
   // the prefix pass, the partitions of the rest of the context follow
   int32_t prefix_blocks, prefix_chunks;
   uint32_t* err;            // the context's misuse word (page ids outside the pool)
-  // vk_append_decode over an I8_BLK pool with the append folded into the decode
-  // (null otherwise): the new K and V rows [n_seqs][n_kv_heads][io_hd] of
-  // fold_dtype, the call's append epoch and the pool's per-tile claim words
+  // vk_append_decode with the append folded into the decode (null otherwise): the new
+  // K and V rows [n_seqs][n_kv_heads][io_hd] of fold_dtype, and over I8_BLK pools the
+  // call's append epoch and the pool's per-tile claim words
   const void* fold_k;
   const void* fold_v;
   int32_t fold_dtype;
