@@ -107,13 +107,15 @@ def rotate(x, pos, style, table):
     return out
 
 
+@pytest.mark.parametrize("n,in_a_row", [(5000, False), (5000, True), (17000, True)])
 @pytest.mark.parametrize("kv", [O.F16, O.I8_BLK])
-def test_append_prompt_of_many_windows(ctx, kv):
-    """A prompt longer than a window of 16 tokens per workgroup, from an offset inside a block."""
-    print(f"append long prompt kv={kv}", flush=True)
+def test_append_prompt_of_many_windows(ctx, kv, n, in_a_row):
+    """A prompt longer than a window of 16 tokens per workgroup, from an offset inside a block, over
+    scattered pages and over pages handed out in order (more than 64 slots in a row, as in large pages)."""
+    print(f"append long prompt kv={kv} n={n} in_a_row={in_a_row}", flush=True)
     r = np.random.default_rng(4200)
-    n, blocks = 5000, 330
-    perm = r.permutation(blocks)
+    blocks = (7 + n) // BS + 10
+    perm = np.arange(blocks) if in_a_row else r.permutation(blocks)
     p = np.arange(7, 7 + n)
     sl = (perm[p // BS] * BS + p % BS).astype(np.int64)
     pool = velokv.Pool(ctx, 1, blocks, BS, HKV, 128, kv)
