@@ -50,12 +50,11 @@ constexpr int64_t kMaxPartWgs = 2048;
 // for longer than the small plan saves: bytes per us of a wave among eight of a
 // workgroup, and among fewer; the merge launch of partitions; what stream-K costs
 // beside its blocks, and for each partial that it leaves of the longest context
-// (its merge reads them in turn). In ns. Fitted to 319 ragged batches, skewed ones (16 to 200
-// sequences, one of 500 to 16,000 tokens and the others of 60 to 500) and evenly
-// spread ones, four KV types:
-// 64 x 8 heads of 200 int8-block tokens, one of 1,000 15.4 us against stream-K's 19.1,
-// one of 2,000 22.1 against 20.2, one of 16,000 122 against 33.6; fp16 one of 500 16.3
-// against 19.8, one of 1,000 22.4 against 20.2.
+// (its merge reads them in turn). In ns. Fitted to 319 ragged batches of four KV types,
+// skewed ones (16 to 200 sequences, one of 500 to 16,000 tokens and the others of 60 to
+// 500) and evenly spread ones: 64 x 8 heads of 200 int8-block tokens, one of 1,000 15.4
+// us against stream-K's 19.1, one of 2,000 22.1 against 20.2, one of 16,000 122 against
+// 33.6; fp16 one of 500 16.3 against 19.8, one of 1,000 22.4 against 20.2.
 constexpr int64_t kWaveRate8 = 5400, kWaveRate = 9000;
 constexpr int64_t kMergeNs = 3400;
 constexpr int64_t kTurnNs = 6000;  // each further turn of workgroups on a CU
